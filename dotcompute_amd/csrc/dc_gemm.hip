@@ -7,14 +7,14 @@
 //   - gemm_f32_dma_kernel<T>: fp32 full tiles (m, n multiples of T = 128, or 64 when 128-tiles
 //     cannot fill the CUs; k a multiple of 32). Direct-to-LDS loads, double-buffered LDS, 4 waves
 //     of (T/2)×(T/2), two workgroups per CU.
-//   - gemm_bf16_big_kernel: bf16 with m, n multiples of 256 and k a multiple of 64. 256×256 macro
-//     tile, direct-to-LDS loads of row-major A and B, B fragments through transposing LDS reads,
-//     8 waves of 128×64, one workgroup per CU.
-//   - gemm_f32_kernel / gemm_bf16_kernel: every other shape (bounds-checked where a tile is
-//     ragged). Block tile 128×128, 4 waves of 64×64; the next tile's global loads go to registers
-//     before the current tile's MFMAs and are stored to the other LDS buffer afterwards, with B
-//     transposed on the way in (Bs[n][k], row pitch BK+4 floats), so a lane's operands for 8
-//     MFMAs are two contiguous, bank-conflict-free 16-byte LDS reads.
+//   - gemm_bf16_kernel<TM, TN, ...>: bf16, every shape. 256×256, 128×128 or 64×64 macro tiles by the
+//     number of tiles; direct-to-LDS loads of row-major A and B where rows are 16-byte aligned,
+//     else loads through registers; B fragments through transposing LDS reads.
+//   - gemm_f32_kernel: fp32 shapes that are not full tiles (bounds-checked). Block tile 128×128 or
+//     64×64, 4 waves; the next tile's global loads go to registers before the current tile's MFMAs
+//     and are stored to the other LDS buffer afterwards, with B transposed on the way in (Bs[n][k],
+//     row pitch BK+4 floats), so a lane's operands for 8 MFMAs are two contiguous,
+//     bank-conflict-free 16-byte LDS reads.
 //
 // Operand layout. For a 32×32 MFMA lane l supplies row (A) / column (B) l % 32 and the k-group
 // h = l / 32; the instruction pairs A and B values by (h, element index), so any assignment of
@@ -41,8 +41,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBM = 128;
-constexpr int kBN = 128;
 constexpr int kThreads = 256;
 constexpr int kGroupM = 8;
 
@@ -392,161 +390,43 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const float* __re
 }
 
 // ---------------------------------------------------------------------------------------------
-// bf16 (inputs as raw bf16 bit patterns), fp32 accumulate
-// ---------------------------------------------------------------------------------------------
-template <int BK>
-struct Bf16Smem {
-  static constexpr int kPitch = BK + 8;  // bf16 elements per LDS row (16-byte aligned rows)
-  unsigned short a[2][kBM][kPitch];
-  unsigned short b[2][kBN][kPitch];
-};
-
-template <int BK, bool CHECKED>
-struct Bf16Loader {
-  // 8 bf16 (16 bytes) per slot.
-  static constexpr int kASlots = kBM * BK / 8 / kThreads;
-  static constexpr int kBSlots = kBN * BK / 8 / kThreads;
-  u16x8 ra[kASlots];
-  u16x8 rb[kBSlots];
-
-  __device__ inline void load(const unsigned short* __restrict__ A, const unsigned short* __restrict__ B, int M, int N,
-                              int K, int m0, int n0, int k0, int tid) {
-#pragma unroll
-    for (int i = 0; i < kASlots; ++i) {
-      const int s = tid + i * kThreads;
-      const int row = s / (BK / 8), kq = s % (BK / 8);
-      const int gm = m0 + row, gk = k0 + 8 * kq;
-      if (!CHECKED) {
-        ra[i] = *reinterpret_cast<const u16x8*>(A + (size_t)gm * K + gk);
-      } else {
-        u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (gm < M) {
-          const unsigned short* p = A + (size_t)gm * K;
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (gk + e < K) v[e] = p[gk + e];
-        }
-        ra[i] = v;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kBSlots; ++i) {
-      const int s = tid + i * kThreads;
-      const int nq = s / BK, k = s % BK;
-      const int gk = k0 + k, gn = n0 + 8 * nq;
-      if (!CHECKED) {
-        rb[i] = *reinterpret_cast<const u16x8*>(B + (size_t)gk * N + gn);
-      } else {
-        u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (gk < K) {
-          const unsigned short* p = B + (size_t)gk * N;
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (gn + e < N) v[e] = p[gn + e];
-        }
-        rb[i] = v;
-      }
-    }
-  }
-
-  __device__ inline void store(Bf16Smem<BK>& sm, int buf, int tid) {
-#pragma unroll
-    for (int i = 0; i < kASlots; ++i) {
-      const int s = tid + i * kThreads;
-      const int row = s / (BK / 8), kq = s % (BK / 8);
-      *reinterpret_cast<u16x8*>(&sm.a[buf][row][8 * kq]) = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < kBSlots; ++i) {
-      const int s = tid + i * kThreads;
-      const int nq = s / BK, k = s % BK;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) sm.b[buf][8 * nq + e][k] = rb[i][e];
-    }
-  }
-};
-
-template <int BK, bool CHECKED>
-__global__ __launch_bounds__(kThreads, 2) void gemm_bf16_kernel(const unsigned short* __restrict__ A,
-                                                                const unsigned short* __restrict__ B,
-                                                                float* __restrict__ C, int M, int N, int K,
-                                                                int tiles_m, int tiles_n) {
-  __shared__ Bf16Smem<BK> sm;
-  const TileCoord tc = map_tile(tiles_m, tiles_n);
-  const int m0 = tc.tm * kBM, n0 = tc.tn * kBN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int r = lane & 31, h = lane >> 5;
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-  Bf16Loader<BK, CHECKED> ld;
-  const int kt_count = (K + BK - 1) / BK;
-  ld.load(A, B, M, N, K, m0, n0, 0, tid);
-  ld.store(sm, 0, tid);
-  __syncthreads();
-
-  for (int kt = 0; kt < kt_count; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < kt_count) ld.load(A, B, M, N, K, m0, n0, (kt + 1) * BK, tid);
-#pragma unroll
-    for (int ks = 0; ks < BK; ks += 16) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-        a[mt] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(&sm.a[buf][wm * 64 + mt * 32 + r][ks + 8 * h]));
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-        b[nt] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(&sm.b[buf][wn * 64 + nt * 32 + r][ks + 8 * h]));
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
-    }
-    if (kt + 1 < kt_count) ld.store(sm, buf ^ 1, tid);
-    __syncthreads();
-  }
-
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const int col = n0 + wn * 64 + nt * 32 + r;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm * 64 + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-        if (!CHECKED || (row < M && col < N)) C[(size_t)row * N + col] = acc[mt][nt][v];
-      }
-    }
-}
-
-// ---------------------------------------------------------------------------------------------
-// bf16, large tiles: C = A·B straight from row-major A[M][K] and B[K][N].
+// bf16 inputs (raw bit patterns), fp32 accumulate: C = A·B straight from row-major A[M][K], B[K][N].
 //
-// Macro tile 256×256, BK = 64, double-buffered LDS (2 × (32 + 32) KiB = 128 KiB, one workgroup
-// per CU). 512 threads as 2×4 waves of 128×64 (4×2 MFMA 32×32×16 tiles, 128 accumulators per
-// lane), two waves per SIMD so one's LDS and barrier waits overlap the other's MFMAs.
+// Macro tile TM×TN, BK = 64, double-buffered LDS, WM×WN waves of 32·kMT × 32·kNT each (MFMA
+// 32×32×16 tiles): 256×256 with 2×4 waves (128 KiB of LDS, one workgroup per CU, 128 accumulators
+// per lane, two waves per SIMD so one's LDS and barrier waits overlap the other's MFMAs), 128×128
+// and 64×64 with 2×2 waves (64 and 32 KiB, two and four workgroups per CU). KS > 1: KS such wave
+// groups per workgroup, each with LDS buffers of its own, take the k tiles in turn (tile kt goes to
+// group kt mod KS), and their sums are added in group order at the end: more loads in flight for a
+// grid of few tiles. Measured with the dispatch in dc_hip_gemm_bf16: 2000×3000×1000 144 -> 21 us
+// (560 TFLOP/s; the kernel it replaces loaded and transposed element by element), 1999×2999×999
+// 31 us; 8192^3 0.84 ms (1300 TFLOP/s), as before. The big tile is bound by the matrix cores' power
+// limit and its tile barriers, the small ones by the latency of one tile's loads per barrier.
 //
-// Global -> LDS: direct-to-LDS loads (buffer_load_dwordx4 ... lds): lane L of a wave's load
-// writes LDS bytes 16·L of a 1 KiB block, so no registers stage the tile and a tile's loads can
-// stay in flight for a whole tile of MFMAs. The swizzles below are applied on the global side:
-// each lane fetches the 16 bytes that belong in its LDS slot.
-// - A tile: 256 rows (m) of 64 k, 128 B per row. The 16-byte k-octet q of row R sits in slot
+// LDS image of a tile, in 1 KiB blocks of 64 16-byte chunks (chunk L of a block is lane L's):
+// - A tile: TM rows (m) of 64 k, 128 B per row. The 16-byte k-octet q of row R sits in slot
 //   q ^ ((R >> 1) & 7), so a fragment read (ds_read_b128: rows R0..R0+15 at one octet for each 16
 //   lanes) touches 16 distinct 16-byte bank groups.
-// - B tile: 64 rows (k) of 256 n, 512 B per row, as B is stored. The 64-byte block b of row k
-//   sits at block b ^ (k & 3). The MFMA wants 8 consecutive k of one column n per lane; the
-//   transposing LDS read ds_read_b64_tr_b16 gives that: within each 16 lanes, source lane
-//   s = 4j + p reads the 4 bf16 of row k0 + j at columns n0 + 4p..4p+3, and lane i receives
-//   B[k0 + j][n0 + i] for j = 0..3 (two such reads give k0..k0+7). The 32 lanes of each half
-//   wave read 4 rows × 64 B at four different 64-byte offsets modulo 256 B: no bank conflicts.
+// - B tile: 64 rows (k) of TN n, 2·TN B per row, as B is stored. The 64-byte block b of row k
+//   sits at block b ^ (k & 3) (TN = 64, two blocks per row: b ^ ((k >> 1) & 1)). The MFMA wants 8
+//   consecutive k of one column n per lane; the transposing LDS read ds_read_b64_tr_b16 gives that:
+//   within each 16 lanes, source lane s = 4j + p reads the 4 bf16 of row k0 + j at columns n0 +
+//   4p..4p+3, and lane i receives B[k0 + j][n0 + i] for j = 0..3 (two such reads give k0..k0+7).
+//   The 32 lanes of each half wave read 4 rows × 64 B at four different 64-byte offsets modulo
+//   256 B: no bank conflicts.
+// The swizzles are applied on the global side: each lane fetches the 16 bytes that belong in its
+// LDS slot.
+//
+// Global -> LDS, two loaders:
+// - kDma (16-byte aligned rows: k and n multiples of 8, aligned operands): direct-to-LDS loads
+//   (buffer_load_dwordx4 ... lds: lane L writes LDS bytes 16·L of a block), so no registers stage
+//   the tile and a tile's loads stay in flight for a whole tile of MFMAs. Rows past M and columns
+//   past N re-read the last ones (their results are not stored); in a last tile of fewer than 64 k
+//   the chunks past K are requested past the buffer range, which loads zeros.
+// - registers (any other shape): 16-byte loads at the elements' own alignment, stored to the same
+//   LDS slots a tile later. A tile past M or N is moved back to end at M or N, so its loads need no
+//   checks (rows and columns that another tile owns are not stored); the last tile of a ragged k,
+//   and matrices smaller than one tile, take element-wise checked loads.
 //
 // Pipeline of tile kt (buffer kt & 1): steps 0..2 run their MFMAs with the next step's fragment
 // reads between them; then the tile's one barrier (which also waits for tile kt+1's loads, issued
@@ -554,82 +434,153 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_bf16_kernel(const unsigned s
 // finished with, and the last step's MFMAs run with tile kt+1's step-0 fragment reads between
 // them, so no LDS latency is exposed after the barrier.
 // ---------------------------------------------------------------------------------------------
-constexpr int kBM2 = 256, kBN2 = 256, kBK2 = 64;
-constexpr int kBigThreads = 512;
-constexpr int kWaveM = 128, kWaveN = 64;       // wave tile
-constexpr int kMT = kWaveM / 32, kNT = kWaveN / 32;
-constexpr int kARow = kBK2 * 2;                // bytes per A row in LDS (64 k)
-constexpr int kBRow = kBN2 * 2;                // bytes per B row in LDS (256 n)
+constexpr int kBK2 = 64;
+constexpr int kARow = kBK2 * 2;  // bytes per A row in LDS (64 k)
 
-struct Bf16BigSmem {
-  unsigned short a[2][kBM2 * kBK2];
-  unsigned short b[2][kBK2 * kBN2];
+template <int TM, int TN>
+struct Bf16Smem {
+  unsigned short a[2][TM * kBK2];
+  unsigned short b[2][kBK2 * TN];
 };
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
+// 8 bf16 at the alignment of one (the unaligned 16-byte load)
+typedef unsigned short u16x8_any __attribute__((ext_vector_type(8), aligned(2)));
 
-// Issues the direct-to-LDS loads of one BK slice (k0..k0+63) of the workgroup's A panel (rows
-// m0..m0+255, buffer resource `ra`) and B panel (columns n0..n0+255 of rows k0.., resource `rb`)
-// into LDS buffer BUF. Wave w's load i fills A rows 8·(8i + w) .. +7 and B rows 2·(8i + w) .. +1
-// (1 KiB each). `avoff` / `bvoff` are the lane's byte offsets inside such a block's global rows;
-// the block's global row offset is uniform (scalar).
-template <int BUF>
-__device__ inline void bf16_tile_to_lds(Bf16BigSmem& sm, __amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, int K,
-                                        int N, int k0, int wave, uint32_t avoff, uint32_t bvoff) {
+// Buffer range of the kDma loader: the host keeps every byte offset below it, so a lane that must
+// load zeros asks for kPastRange, whatever the uniform offset added to it.
+constexpr int32_t kDmaRange = 0x7FFFFFFF;
+constexpr uint32_t kPastRange = 0x80000000u;
+
+// Issues the direct-to-LDS loads of the k tile at k0 (klim = k rows left from there) for the panels
+// that start at A (row pitch K, in avoff) and B (row pitch N). Wave w's load i fills block i·WAVES + w
+// of the A and of the B tile; avoff[i] / bvoff are the lane's byte offsets within the panel and the
+// block's rows, the uniform part is the scalar offset.
+template <int ABLOCKS, int BBLOCKS, int WAVES, int ROWS>
+__device__ inline void bf16_tile_to_lds(unsigned short* la, unsigned short* lb, const unsigned short* __restrict__ A,
+                                        const unsigned short* __restrict__ B, int N, int k0, int klim, int wave, int akq,
+                                        const uint32_t* avoff, int brow, uint32_t bvoff) {
+  const auto ra = dc::range_rsrc(A, kDmaRange), rb = dc::range_rsrc(B, kDmaRange);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int blk = 8 * i + wave;
-    const int32_t asoff = (8 * blk * K + k0) * (int32_t)sizeof(unsigned short);
-    const int32_t bsoff = (k0 + 2 * blk) * N * (int32_t)sizeof(unsigned short);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)&sm.a[BUF][blk * 512], 16, avoff, asoff, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)&sm.b[BUF][blk * 512], 16, bvoff, bsoff, 0, 0);
+  for (int i = 0; i < ABLOCKS; ++i)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(la + (i * WAVES + wave) * 512), 16,
+                                             akq < klim ? avoff[i] : kPastRange, k0 * 2, 0, 0);
+#pragma unroll
+  for (int i = 0; i < BBLOCKS; ++i) {
+    const int krow = ROWS * (i * WAVES + wave);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(lb + (i * WAVES + wave) * 512), 16,
+                                             krow + brow < klim ? bvoff : kPastRange, (k0 + krow) * N * 2, 0, 0);
   }
 }
 
-__global__ __launch_bounds__(kBigThreads, 1) void gemm_bf16_big_kernel(const unsigned short* __restrict__ A,
-                                                                       const unsigned short* __restrict__ B,
-                                                                       float* __restrict__ C, int M, int N, int K,
-                                                                       int tiles_m, int tiles_n) {
-  __shared__ __align__(16) Bf16BigSmem sm;  // 128 KiB of static LDS (gfx950 has 160 KiB per CU)
+template <int TM, int TN, int WM, int WN, int KS, bool kDma>
+__global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gemm_bf16_kernel(
+    const unsigned short* __restrict__ A, const unsigned short* __restrict__ B, float* __restrict__ C, int M, int N,
+    int K, int tiles_m, int tiles_n) {
+  constexpr int kWaves = WM * WN;
+  constexpr int kMT = TM / WM / 32, kNT = TN / WN / 32;  // MFMA tiles per wave
+  constexpr int kABlocks = TM / 8 / kWaves, kBBlocks = TN / 8 / kWaves;  // 1 KiB blocks per wave and tile
+  constexpr int kRows = 512 / TN;    // k-rows of B per block
+  constexpr int kBRow = 2 * TN;      // bytes per B row in LDS
+  using Smem = Bf16Smem<TM, TN>;
+  __shared__ __align__(16) Smem sms[KS];
   const TileCoord tc = map_tile(tiles_m, tiles_n);
-  const int m0 = tc.tm * kBM2, n0 = tc.tn * kBN2;
+  const int m0 = tc.tm * TM;
+  // (register loader: the last tile ends at N where N holds a whole tile)
+  const int n0 = kDma || N < TN ? tc.tn * TN : min(tc.tn * TN, N - TN);
   // wave index in a scalar register: the loads' LDS bases and scalar offsets derive from it
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / (kBN2 / kWaveN), wn = wave % (kBN2 / kWaveN);
+  const int tid = threadIdx.x, lane = tid & 63, gwave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = gwave / kWaves, wave = gwave % kWaves;
+  Smem& sm = sms[group];
+  const int wm = wave / WN, wn = wave % WN;
   const int r = lane & 31, h = lane >> 5;
-  // load side: A panel (256 rows of K) and B panel (K rows, 256 columns at row pitch N) as buffer
-  // ranges (both < 2 GiB, checked by the host)
-  const auto ra = dc::range_rsrc(A + (size_t)m0 * K, kBM2 * K * (int32_t)sizeof(unsigned short));
-  const auto rb = dc::range_rsrc(B + n0, ((K - 1) * N + kBN2) * (int32_t)sizeof(unsigned short));
-  // A: lane -> row L / 8 of the block, slot L % 8 = octet (L % 8) ^ ((row >> 1) % 8), where
-  // (row >> 1) % 8 depends on w and L only
+  const int kt_count = ((K + kBK2 - 1) / kBK2 + KS - 1) / KS;  // k tiles per group
+  auto bswz = [](int k) __attribute__((always_inline)) { return TN == 64 ? (k >> 1) & 1 : k & 3; };
+
+  // ---- load side. A: lane -> row L / 8 of a block, slot L % 8 = octet (L % 8) ^ ((row >> 1) % 8),
+  // the same for each of the wave's blocks i·waves + w. B: lane -> row L / (TN / 8) of the block and
+  // chunk L % (TN / 8), which holds the global chunk of the swizzle.
   const int arow = lane >> 3;
-  const int aswz = ((8 * wave + arow) >> 1) & 7;
-  const uint32_t avoff = (uint32_t)((arow * K + 8 * ((lane & 7) ^ aswz)) * (int)sizeof(unsigned short));
-  // B: lane -> row L / 32 of the block pair, 16-byte slot c = L % 32 (64-byte block c / 4), which
-  // holds global chunk 4·((c / 4) ^ (row & 3)) + c % 4; row & 3 = (2w + L / 32) & 3
-  const int brow = lane >> 5, bc = lane & 31;
-  const int bchunk = 4 * ((bc >> 2) ^ ((2 * wave + brow) & 3)) + (bc & 3);
-  const uint32_t bvoff = (uint32_t)((brow * N + 8 * bchunk) * (int)sizeof(unsigned short));
-  // read side, A: fragment rows R = 32·t + r (t: wave and tile offsets, multiples of 32), so the
-  // swizzle is (r >> 1) % 8; k-octet 2·step + h. Byte offsets of step s in buffer 0 (buffer and mt
-  // offsets are immediates).
+  const int akq = 8 * ((lane & 7) ^ ((4 * wave + (arow >> 1)) & 7));
+  const int brow = lane / (TN / 8), bc = lane % (TN / 8);
+  const int bchunk = 4 * ((bc >> 2) ^ bswz(kRows * wave + brow)) + (bc & 3);
+  uint32_t avoff[kABlocks], bvoff = 0;
+  u16x8 sa[kABlocks], sb[kBBlocks];
+  if constexpr (kDma) {
+#pragma unroll
+    for (int i = 0; i < kABlocks; ++i)
+      avoff[i] = (uint32_t)((min(8 * (i * kWaves + wave) + arow, M - 1 - m0) * K + akq) * 2);
+    bvoff = (uint32_t)((brow * N + min(8 * bchunk, N - 8 - n0)) * 2);
+  }
+  // Loads the group's k tile KT (into LDS buffer BUF, or into registers).
+  auto load_tile = [&](auto BUF, int KT) __attribute__((always_inline)) {
+    constexpr int kBuf = decltype(BUF)::value;
+    const int k0 = (KT * KS + group) * kBK2;
+    const int klim = K - k0;  // k rows of the tile that exist (64 or more: all; none: the tile is zero)
+    if constexpr (kDma) {
+      bf16_tile_to_lds<kABlocks, kBBlocks, kWaves, kRows>(sm.a[kBuf], sm.b[kBuf], A + (size_t)m0 * K, B + n0, N, k0, klim,
+                                                          wave, akq, avoff, brow, bvoff);
+    } else {
+      const bool whole_k = klim >= kBK2;  // uniform, as is N >= TN
+      if (whole_k) {
+#pragma unroll
+        for (int i = 0; i < kABlocks; ++i)
+          sa[i] = *reinterpret_cast<const u16x8_any*>(A + (size_t)min(m0 + 8 * (i * kWaves + wave) + arow, M - 1) * K +
+                                                      k0 + akq);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kABlocks; ++i) {
+          const unsigned short* p = A + (size_t)min(m0 + 8 * (i * kWaves + wave) + arow, M - 1) * K + k0 + akq;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) sa[i][e] = akq + e < klim ? p[e] : 0;
+        }
+      }
+      if (whole_k && N >= TN) {
+#pragma unroll
+        for (int i = 0; i < kBBlocks; ++i)
+          sb[i] = *reinterpret_cast<const u16x8_any*>(B + (size_t)(k0 + kRows * (i * kWaves + wave) + brow) * N + n0 +
+                                                      8 * bchunk);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kBBlocks; ++i) {
+          const int gk = kRows * (i * kWaves + wave) + brow, gn = n0 + 8 * bchunk;
+          const unsigned short* p = B + (size_t)(k0 + gk) * N + gn;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) sb[i][e] = gk < klim && gn + e < N ? p[e] : 0;
+        }
+      }
+    }
+  };
+  // Register loader: stores the loaded tile into LDS buffer BUF.
+  auto store_tile = [&](auto BUF) __attribute__((always_inline)) {
+    constexpr int kBuf = decltype(BUF)::value;
+#pragma unroll
+    for (int i = 0; i < kABlocks; ++i)
+      *reinterpret_cast<u16x8*>(&sm.a[kBuf][(i * kWaves + wave) * 512 + lane * 8]) = sa[i];
+#pragma unroll
+    for (int i = 0; i < kBBlocks; ++i)
+      *reinterpret_cast<u16x8*>(&sm.b[kBuf][(i * kWaves + wave) * 512 + lane * 8]) = sb[i];
+  };
+
+  // ---- read side, A: fragment rows R = 32·t + r (t: wave and tile offsets), so the swizzle is
+  // (r >> 1) % 8; k-octet 2·step + h. Byte offsets of step s in buffer 0 (buffer and mt offsets are
+  // immediates).
   const int rswz = (r >> 1) & 7;
   uint32_t aoff[4];
 #pragma unroll
   for (int st = 0; st < 4; ++st)
-    aoff[st] = (uint32_t)(wm * kWaveM + r) * kARow + 16u * (uint32_t)((2 * st + h) ^ rswz);
+    aoff[st] = (uint32_t)(wm * 32 * kMT + r) * kARow + 16u * (uint32_t)((2 * st + h) ^ rswz);
   // read side, B: source lane s = L % 16 = 4j + p reads row 8h + j (+16·step, +4 for the upper
-  // four k: immediates) at columns wn·64 + nt·32 + 16·((L / 16) & 1) + 4p, whose 64-byte block
-  // 2·wn + nt sits at (2·wn + nt) ^ j since the row is ≡ j (mod 4)
+  // four k: immediates) at columns wn·32·kNT + nt·32 + 16·((L / 16) & 1) + 4p; the row is ≡ j
+  // (mod 4), so its 64-byte block kNT·wn + nt sits at block ^ bswz(j)
   uint32_t boff[kNT];
   {
     const int j = (lane & 15) >> 2, p4 = lane & 3, cg = (lane >> 4) & 1;
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt)
-      boff[nt] = (uint32_t)offsetof(Bf16BigSmem, b) + (uint32_t)((8 * h + j) * kBRow) +
-                 64u * (uint32_t)((2 * wn + nt) ^ j) + (uint32_t)(32 * cg + 8 * p4);
+      boff[nt] = (uint32_t)offsetof(Smem, b) + (uint32_t)((8 * h + j) * kBRow) +
+                 64u * (uint32_t)((kNT * wn + nt) ^ bswz(j)) + (uint32_t)(32 * cg + 8 * p4);
   }
 
   f32x16 acc[kMT][kNT];
@@ -642,7 +593,6 @@ __global__ __launch_bounds__(kBigThreads, 1) void gemm_bf16_big_kernel(const uns
 
   constexpr int kSteps = kBK2 / 16;
   static_assert(kSteps == 4, "four 16-wide k steps per tile");
-  const int kt_count = K / kBK2;
   const unsigned char* lds = reinterpret_cast<const unsigned char*>(&sm);
   // B fragments of a whole tile (4 steps × kNT × 2 transposing reads) in one burst. The compiler
   // cannot tell these intrinsic reads apart from the LDS the direct-to-LDS loads write, so it
@@ -661,7 +611,7 @@ __global__ __launch_bounds__(kBigThreads, 1) void gemm_bf16_big_kernel(const uns
       }
   };
   auto read_a = [&](auto BUF, int step, bf16x8* a) __attribute__((always_inline)) {
-    constexpr uint32_t kBufA = (uint32_t)decltype(BUF)::value * kBM2 * kARow;
+    constexpr uint32_t kBufA = (uint32_t)decltype(BUF)::value * TM * kARow;
 #pragma unroll
     for (int mt = 0; mt < kMT; ++mt)
       a[mt] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(lds + aoff[step] + kBufA + mt * 32 * kARow));
@@ -681,12 +631,23 @@ __global__ __launch_bounds__(kBigThreads, 1) void gemm_bf16_big_kernel(const uns
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
     }
   };
+  // The next tile is in LDS and every wave is done reading the other buffer.
+  auto tile_barrier = [&](auto NEXT) __attribute__((always_inline)) {
+    if constexpr (kDma) {
+      dma_barrier();
+    } else {
+      store_tile(NEXT);
+      __syncthreads();
+    }
+  };
   bf16x8 fa[2][kMT], fb[2][kSteps][kNT];
-  bf16_tile_to_lds<0>(sm, ra, rb, K, N, 0, wave, avoff, bvoff);
-  dma_barrier();
-  read_b_tile(std::integral_constant<int, 0>{}, fb[0]);
-  read_a(std::integral_constant<int, 0>{}, 0, fa[0]);
-  if (kt_count > 1) bf16_tile_to_lds<1>(sm, ra, rb, K, N, kBK2, wave, avoff, bvoff);
+  constexpr std::integral_constant<int, 0> kBuf0{};
+  constexpr std::integral_constant<int, 1> kBuf1{};
+  load_tile(kBuf0, 0);
+  tile_barrier(kBuf0);
+  read_b_tile(kBuf0, fb[0]);
+  read_a(kBuf0, 0, fa[0]);
+  if (kt_count > 1) load_tile(kBuf1, 1);
   // Tile kt in LDS buffer BUF = kt % 2 (the loop is unrolled by two, so buffer offsets are
   // constants; a macro rather than a lambda keeps the fragment arrays plain registers).
 #define DC_BF16_TILE(BUF, KT)                                                                      \
@@ -694,25 +655,24 @@ __global__ __launch_bounds__(kBigThreads, 1) void gemm_bf16_big_kernel(const uns
     _Pragma("unroll") for (int step = 0; step + 1 < kSteps; ++step) {                              \
       const int cur = step & 1;                                                                    \
       __builtin_amdgcn_sched_barrier(0);                                                           \
-      read_a(std::integral_constant<int, BUF>{}, step + 1, fa[cur ^ 1]);                           \
+      read_a(kBuf##BUF, step + 1, fa[cur ^ 1]);                                                    \
       mfmas(fa[cur], fb[BUF][step]);                                                               \
       interleave_reads();                                                                          \
       __builtin_amdgcn_sched_barrier(0);                                                           \
     }                                                                                              \
     /* tile KT+1 is in LDS; every wave is done reading buffer BUF (after the last tile the */     \
     /* barrier and the reads of the other buffer are harmless and unused) */                      \
-    dma_barrier();                                                                                 \
+    tile_barrier(std::integral_constant<int, 1 - (BUF)>{});                                        \
     read_b_tile(std::integral_constant<int, 1 - (BUF)>{}, fb[1 - (BUF)]);                          \
-    if ((KT) + 2 < kt_count)                                                                       \
-      bf16_tile_to_lds<BUF>(sm, ra, rb, K, N, ((KT) + 2) * kBK2, wave, avoff, bvoff);              \
+    if ((KT) + 2 < kt_count) load_tile(kBuf##BUF, (KT) + 2);                                       \
     __builtin_amdgcn_sched_barrier(0);                                                             \
     read_a(std::integral_constant<int, 1 - (BUF)>{}, 0, fa[0]);                                    \
     mfmas(fa[1], fb[BUF][kSteps - 1]);                                                             \
     interleave_reads();                                                                            \
     __builtin_amdgcn_sched_barrier(0);                                                             \
   }
-  // K is a positive multiple of 64 (host check): at least one tile, and no zero-trip path that
-  // would keep the accumulators' initial values live beside the loop
+  // K > 0 (host check): at least one tile, and no zero-trip path that would keep the accumulators'
+  // initial values live beside the loop
   __builtin_assume(kt_count > 0);
   int kt = 0;
   do {
@@ -722,16 +682,35 @@ __global__ __launch_bounds__(kBigThreads, 1) void gemm_bf16_big_kernel(const uns
   } while (kt < kt_count);
 #undef DC_BF16_TILE
 
+  if constexpr (KS > 1) {  // the groups' sums, added in group order by group 0
+    static_assert(sizeof(Smem) >= kWaves * 64 * kMT * kNT * 16 * sizeof(float), "a group's sums fit in its buffers");
+    float* part = reinterpret_cast<float*>(&sm) + tid % (64 * kWaves);
+    __syncthreads();
+    if (group > 0)
+#pragma unroll
+      for (int i = 0; i < kMT * kNT * 16; ++i) part[i * 64 * kWaves] = acc[i / 16 / kNT][i / 16 % kNT][i % 16];
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g = 1; g < KS; ++g) {
+      const float* other = reinterpret_cast<const float*>(&sms[g]) + tid;
+#pragma unroll
+      for (int i = 0; i < kMT * kNT * 16; ++i) acc[i / 16 / kNT][i / 16 % kNT][i % 16] += other[i * 64 * kWaves];
+    }
+  }
   // acc[mt][nt][v] holds C[row][col], row = 8*(v/4) + 4*h + v%4, col = r (within the 32×32 tile).
+  // Only the rows and columns of this tile's own place are stored.
+  const bool whole = m0 + TM <= M && n0 + TN <= N && n0 == tc.tn * TN;
 #pragma unroll
   for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt) {
-      const int col = n0 + wn * kWaveN + nt * 32 + r;
+      const int col = n0 + (wn * kNT + nt) * 32 + r;
+      const bool cok = col < N && col >= tc.tn * TN;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm * kWaveM + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-        C[(size_t)row * N + col] = acc[mt][nt][v];
+        const int row = m0 + (wm * kMT + mt) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+        if (whole || (cok && row < M)) C[(size_t)row * N + col] = acc[mt][nt][v];
       }
     }
 }
@@ -755,7 +734,14 @@ __global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float* __restric
 }
 
 constexpr int kBKf32 = 32;
-constexpr int kBKbf16 = 64;
+
+template <int TM, int TN, int WM, int WN, int KS, bool kDma>
+void launch_bf16(dc_hip_ctx* ctx, const unsigned short* a, const unsigned short* b, float* c, int64_t m, int64_t n,
+                 int64_t k) {
+  const int tiles_m = (int)((m + TM - 1) / TM), tiles_n = (int)((n + TN - 1) / TN);
+  gemm_bf16_kernel<TM, TN, WM, WN, KS, kDma><<<(unsigned)(tiles_m * tiles_n), 64 * WM * WN * KS, 0, ctx->stream>>>(
+      a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
+}
 
 int32_t check_dims(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k < 0) return DC_ERR_INVALID_ARGUMENT;
@@ -805,24 +791,37 @@ DC_HIP_API int32_t dc_hip_gemm_bf16(dc_hip_ctx* ctx, const uint16_t* a, const ui
   if (!c || (k > 0 && (!a || !b))) return DC_ERR_INVALID_ARGUMENT;
   DC_CTX_ENTER(ctx);
   if (k == 0) return dc::zero_async(ctx, c, (size_t)(m * n) * sizeof(float));
-  const int tiles_m = (int)((m + kBM - 1) / kBM), tiles_n = (int)((n + kBN - 1) / kBN);
-  const unsigned grid = (unsigned)(tiles_m * tiles_n);
   const unsigned short* A = reinterpret_cast<const unsigned short*>(a);
   const unsigned short* B = reinterpret_cast<const unsigned short*>(b);
-  // large tiles: the A panel (256 rows of k bf16) and the B panel (k rows at pitch n) as buffer
-  // ranges, each < 2 GiB
-  if ((m % kBM2 == 0) && (n % kBN2 == 0) && (k % kBK2 == 0) && dc::aligned16(a) && dc::aligned16(b) &&
-      (int64_t)k * kBM2 * 2 < ((int64_t)1 << 31) && (int64_t)k * n * 2 < ((int64_t)1 << 31)) {
-    const int tm2 = (int)(m / kBM2), tn2 = (int)(n / kBN2);
-    gemm_bf16_big_kernel<<<(unsigned)(tm2 * tn2), kBigThreads, 0, ctx->stream>>>(
-        A, B, c, (int)m, (int)n, (int)k, tm2, tn2);
-    return dc::last_launch_status();
+  // 16-byte rows, and every byte offset of the panels (256 rows of A; B's rows, with up to four k
+  // tiles past the last) inside the buffer range: the direct-to-LDS loader
+  const bool dma = n % 8 == 0 && k % 8 == 0 && dc::aligned16(a) && dc::aligned16(b) &&
+                   (k + 4 * kBK2) * 256 * 2 < (int64_t)kDmaRange && (k + 4 * kBK2) * n * 2 < (int64_t)kDmaRange;
+  // The widest tile that still gives the chip enough workgroups; then, where even the small tiles
+  // leave CUs idle, a k dimension split over the wave groups of a workgroup. Measured (us, direct-to-LDS
+  // loader, tiles 256 / 128 / 64; "x2", "x4": that many k groups):
+  //   3072x3072x1024 (144 tiles of 256): 27.5 / 32.6 / 33.8;  2048x8192x512 (256): 24.1 / 26.5 / 31.4
+  //   2000x3000x1000 (96 tiles of 256, 384 of 128): 29.0 / 21.2 / 28.8
+  //   2048^3 (256 of 128): 45.2 / 28.2 (x2 23.7) / 27.3;  1536^3 (144): 34.6 / 20.3 (x2 17.5) / 15.2
+  //   256x8192x8192 (512 of 64): 151 / 80 / 61, x2 51.8, x4 66;  1024^3 (256 of 64): 7.4, x2 6.6, x4 6.7
+  //   64x8192x8192 (128 of 64): 61, x2 43, x4 36;  512x512x4096 (64 of 64): 32, x2 24, x4 20
+  //   512^3: 4.6, x2 4.4, x4 4.9
+  // Register loader (128 / 64): 2047^3 42 / 52, 1535^3 33 / 29, 1023^3 21 / 12.4 (x4 11.0),
+  // 511x511x4095 61 / 48 (x4 32).
+  const int64_t cus = std::max(1, ctx->cu_count);
+  auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
+  if (dma) {
+    if (2 * tiles(256) > cus) launch_bf16<256, 256, 2, 4, 1, true>(ctx, A, B, c, m, n, k);
+    else if (tiles(128) > cus) launch_bf16<128, 128, 2, 2, 1, true>(ctx, A, B, c, m, n, k);
+    else if (4 * tiles(128) > 3 * cus) launch_bf16<128, 128, 2, 2, 2, true>(ctx, A, B, c, m, n, k);
+    else if (tiles(64) > 2 * cus || k < 512) launch_bf16<64, 64, 2, 2, 1, true>(ctx, A, B, c, m, n, k);
+    else if (2 * tiles(64) > cus || k < 2048) launch_bf16<64, 64, 2, 2, 2, true>(ctx, A, B, c, m, n, k);
+    else launch_bf16<64, 64, 2, 2, 4, true>(ctx, A, B, c, m, n, k);
+  } else {
+    if (n >= 128 && 4 * tiles(128) > 3 * cus) launch_bf16<128, 128, 2, 2, 1, false>(ctx, A, B, c, m, n, k);
+    else if (tiles(64) > cus || k < 1000) launch_bf16<64, 64, 2, 2, 1, false>(ctx, A, B, c, m, n, k);
+    else launch_bf16<64, 64, 2, 2, 4, false>(ctx, A, B, c, m, n, k);
   }
-  const bool full = (m % kBM == 0) && (n % kBN == 0) && (k % kBKbf16 == 0) && dc::aligned16(a) && dc::aligned16(b);
-  if (full)
-    gemm_bf16_kernel<kBKbf16, false><<<grid, kThreads, 0, ctx->stream>>>(A, B, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
-  else
-    gemm_bf16_kernel<kBKbf16, true><<<grid, kThreads, 0, ctx->stream>>>(A, B, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
   return dc::last_launch_status();
 }
 

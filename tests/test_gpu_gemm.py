@@ -169,3 +169,26 @@ def test_convert_f32_to_bf16_bit_exact(ctx):
     assert np.array_equal(got, ref)
     ctx.free(d)
     ctx.free(o)
+
+
+# One shape or two per tile choice of the bf16 dispatch (on 256 CUs), each with ragged rows, columns
+# and a last k tile that is not whole. 16-byte rows: 256-tiles, 128-tiles, 128-tiles with two k groups,
+# 64-tiles with one, two and four; other rows: 128-tiles, 64-tiles with one and four k groups,
+# fewer columns than a tile.
+@pytest.mark.parametrize("shape", [(2824, 3080, 72), (2200, 2056, 200), (1800, 1912, 136), (200, 264, 200), (8, 8, 8),
+                                   (456, 520, 520), (72, 136, 2120), (1799, 1911, 137), (63, 65, 129), (300, 50, 70),
+                                   (129, 131, 1001), (70, 9, 64)])
+def test_gemm_bf16_ragged_tiles(ctx, shape):
+    m, n, k = shape
+    a, b = make_inputs(m, n, k)
+    a = oracle.bf16_to_f32(oracle.f32_to_bf16(a)).reshape(m, k)
+    b = oracle.bf16_to_f32(oracle.f32_to_bf16(b)).reshape(k, n)
+    c = run_gemm(ctx, a, b, kind="bf16")
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    absref = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    # products of bf16 values are exact in float32; k additions, each within one float32 ulp
+    assert np.all(np.abs(c - ref) <= k * 2.0 ** -23 * absref)
+    # what lies past a row's end (the next row, here of infinities) reaches no result
+    a[1:] = np.inf
+    c0 = run_gemm(ctx, a, b, kind="bf16")[0]
+    assert np.array_equal(c0, c[0])
