@@ -1,20 +1,19 @@
 // dc_gemm.hip — dense row-major GEMM C[m×n] = A[m×k]·B[k×n] on the gfx950 matrix cores.
 //
-// fp32: v_mfma_f32_32x32x2_f32 (fp32 inputs, fp32 accumulate).
+// fp32: three bf16 pieces per value on v_mfma_f32_32x32x16_bf16, or v_mfma_f32_32x32x2_f32 (fp32
+// accumulate in both).
 // bf16: v_mfma_f32_32x32x16_bf16 (bf16 inputs, fp32 accumulate).
 //
 // Kernels, by the shapes that take them:
-//   - gemm_f32_dma_kernel<T>: fp32 full tiles (m, n multiples of T = 128, or 64 when 128-tiles
-//     cannot fill the CUs; k a multiple of 32). Direct-to-LDS loads, double-buffered LDS, 4 waves
-//     of (T/2)×(T/2), two workgroups per CU.
+//   - gemm_f32_split_kernel<TM, TN, ...>: fp32, by six bf16 products per fp32 product; 256×256,
+//     128×128 or 64×64 macro tiles by the number of tiles.
+//   - gemm_f32_dma_kernel<64>: fp32 full 64-tiles, few of them with a short k, on the fp32
+//     instructions: direct-to-LDS loads, double-buffered LDS, 4 waves of 32×32.
+//   - gemm_f32_kernel: the fp32 shapes left (fewer than 64 columns, one or two k tiles),
+//     bounds-checked 64×64 tiles on the fp32 instructions.
 //   - gemm_bf16_kernel<TM, TN, ...>: bf16, every shape. 256×256, 128×128 or 64×64 macro tiles by the
 //     number of tiles; direct-to-LDS loads of row-major A and B where rows are 16-byte aligned,
 //     else loads through registers; B fragments through transposing LDS reads.
-//   - gemm_f32_kernel: fp32 shapes that are not full tiles (bounds-checked). Block tile 128×128 or
-//     64×64, 4 waves; the next tile's global loads go to registers before the current tile's MFMAs
-//     and are stored to the other LDS buffer afterwards, with B transposed on the way in (Bs[n][k],
-//     row pitch BK+4 floats), so a lane's operands for 8 MFMAs are two contiguous,
-//     bank-conflict-free 16-byte LDS reads.
 //
 // Operand layout. For a 32×32 MFMA lane l supplies row (A) / column (B) l % 32 and the k-group
 // h = l / 32; the instruction pairs A and B values by (h, element index), so any assignment of
@@ -30,6 +29,7 @@
 
 #include <cstddef>
 #include <type_traits>
+#include <utility>
 
 #include "dc_device.hpp"
 #include "dc_internal.hpp"
@@ -62,7 +62,8 @@ __device__ inline TileCoord map_tile(int tiles_m, int tiles_n) {
 
 // ---------------------------------------------------------------------------------------------
 // fp32, full tiles (m, n multiples of T, k a multiple of 32): direct-to-LDS loads, no staging
-// registers and no transposing LDS stores.
+// registers and no transposing LDS stores. Launched with T = 64 for grids of at most one tile per CU
+// and k <= 1024 (1024^3: 19.7 us; see the dispatch).
 //   A tile [T rows][32 k] (128 B rows, unpadded): the 16-byte k-quad q of row R sits in slot
 //   q ^ ((R >> 1) & 7), so a fragment read (16 lanes = rows R0..R0+15 at one quad) touches 16
 //   distinct 16-byte bank groups.
@@ -235,8 +236,11 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_dma_kernel(const float* 
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp32. T = macro tile (128, or 64 when 128-tiles cannot occupy the CUs: 1024² has only 64 of
-// them); 4 waves as 2×2, each wave (T/2)×(T/2) = (T/64)×(T/64) MFMA 32×32 tiles.
+// fp32, bounds-checked. T = macro tile; 4 waves as 2×2, each wave (T/2)×(T/2) = (T/64)×(T/64) MFMA
+// 32×32 tiles. The next tile's global loads go to registers before the current tile's MFMAs and are
+// stored to the other LDS buffer afterwards, with B transposed on the way in (Bs[n][k], row pitch
+// BK + 4 floats), so a lane's operands for 8 MFMAs are two contiguous, bank-conflict-free 16-byte
+// LDS reads.
 // ---------------------------------------------------------------------------------------------
 template <int BK, int T>
 struct F32Smem {
@@ -715,6 +719,445 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// fp32 on the bf16 matrix cores: every fp32 value is the exact sum of three bf16 pieces,
+// x = x0 + x1 + x2 (x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1: 8 + 8 + 8 bits, rounded to
+// nearest, so |x1| <= 2^-9 |x| and |x2| <= 2^-18 |x|), and a·b is formed from the six products
+// a0 b0, a0 b1, a1 b0, a0 b2, a1 b1, a2 b0, each exact in fp32; the three left out are below
+// 2^-26 |a b|. 6 bf16 products cost 6/16 of one fp32 product on this chip's matrix cores, and a
+// 32×32×16 instruction adds 16 products per rounding where the fp32 one adds 2, so the result is
+// both faster and closer to the float64 product than the fp32 instructions' (relative error at
+// 8192^3 with normal inputs: 1.4e-6 against 1.6e-6). Measured: 8192^3 7.31 -> 4.50 ms (244
+// TFLOP/s where the fp32 instructions peak at 157), 4096^3 925 -> 561 us, 1537×2049×1023 144 -> 46 us.
+// Bound by the matrix cores at the clock that power allows (the 256-tile) and by what a workgroup's
+// barriers leave uncovered (the small tiles).
+//
+// Where the pieces do not hold the value: infinities and NaN (x - x0 is NaN, so the sum is), values
+// that round up to infinity in bf16 (likewise), and nonzero magnitudes below kSplitMin, whose lowest
+// pieces fall below bf16's subnormals (an error below 2^-134 each). A tile whose sums are not all
+// finite, or that met such small values and has a sum they could have moved by more than 2^-26 of
+// itself, computes itself again with v_mfma_f32_32x32x2_f32 (f32_tile_direct below), so those inputs
+// give what the fp32 instructions give. (8192^3 with every value of A near 2^-110: 10.7 ms against
+// 7.3 ms on the fp32 instructions alone; with a tenth of them scattered: 5.3 ms.) bf16 subnormals and
+// products down to the fp32 subnormals are kept by the matrix cores (measured), so results near
+// 2^-126 are as exact as before.
+//
+// Macro tile TM×TN, KS groups of WM×WN waves that take the k tiles (16 k each) in turn (as
+// gemm_bf16_kernel). A tile's fp32 elements come through registers (16-byte loads at 4-byte alignment,
+// D tiles ahead: so no shape or alignment needs another kernel), are split and stored to LDS as three
+// bf16 planes, in the other of two buffers, while this tile's products run: about 7 VALU
+// instructions per element beside 48 (256-tile) or 24 MFMAs per wave and tile. LDS images per plane:
+// - A: rows of 16 k (32 B); the 16-byte half h of row R sits at h ^ ((R >> 3) & 1), so a
+//   fragment read (16 rows at one half for each 16 lanes) touches 16 distinct 16-byte bank groups.
+// - B: k rows of TN n with the 64-byte blocks swizzled, read through ds_read_b64_tr_b16
+//   (as gemm_bf16_kernel).
+// ---------------------------------------------------------------------------------------------
+constexpr float kSplitMin = 0x1p-102f;
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// Calls f(std::integral_constant<int, I>) for I = 0, 1, ...: a compile-time unrolled loop.
+template <typename F, int... I>
+__device__ __attribute__((always_inline)) inline void for_each_index(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+// The three bf16 pieces of four values, packed; *tiny becomes the smallest (2|x| as bits) - 1 seen
+// (all ones for x = 0).
+__device__ inline void split_quad(dc::f32x4 x, u32x2 (&piece)[3], uint32_t* tiny) {
+  f32x2 v[2] = {{x.x, x.y}, {x.z, x.w}};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t t0 = (__builtin_bit_cast(uint32_t, v[i].x) << 1) - 1u;
+    const uint32_t t1 = (__builtin_bit_cast(uint32_t, v[i].y) << 1) - 1u;
+    *tiny = min(*tiny, min(t0, t1));
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v[i], bf16x2));
+      piece[p][i] = w;
+      if (p < 2) {
+        v[i].x -= __builtin_bit_cast(float, w << 16);
+        v[i].y -= __builtin_bit_cast(float, w & 0xFFFF0000u);
+      }
+    }
+  }
+}
+
+// One workgroup's C tile with the fp32 matrix instructions, into acc (waves of group 0; every wave of the
+// workgroup takes part in the barriers). Operands are staged k-row by k-row in LDS (`la`: 16 rows
+// of TM + 32, `lb`: 16 rows of TN + 32 floats); every load is checked.
+template <int TM, int TN, int kMT, int kNT, int kThreadsPerGroup>
+__device__ __attribute__((always_inline)) inline void f32_tile_direct(const float* __restrict__ A, const float* __restrict__ B, int M,
+                                                          int N, int K, int m0, int n0, int t, bool active, int wm,
+                                                          int wn, float* la, float* lb, f32x16 (&acc)[kMT][kNT]) {
+  constexpr int kA = TM * 16 / kThreadsPerGroup, kB = TN * 16 / kThreadsPerGroup;
+  constexpr int kPitchA = TM + 32, kPitchB = TN + 32;
+  const int lane = t & 63, r = lane & 31, h = lane >> 5;
+  float ea[kA], eb[kB];
+  auto load = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kA; ++i) {
+      const int e = i * kThreadsPerGroup + t, m = m0 + e / 16, k = k0 + e % 16;
+      ea[i] = active && m < M && k < K ? A[(size_t)m * K + k] : 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+      const int e = i * kThreadsPerGroup + t, k = k0 + e / TN, n = n0 + e % TN;
+      eb[i] = active && k < K && n < N ? B[(size_t)k * N + n] : 0.0f;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < kMT * kNT; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[i / kNT][i % kNT][v] = 0.0f;
+  load(0);
+#pragma unroll 1
+  for (int k0 = 0; k0 < K; k0 += 16) {
+    __syncthreads();
+    if (active) {
+#pragma unroll
+      for (int i = 0; i < kA; ++i) {
+        const int e = i * kThreadsPerGroup + t;
+        la[(e % 16) * kPitchA + e / 16] = ea[i];
+      }
+#pragma unroll
+      for (int i = 0; i < kB; ++i) {
+        const int e = i * kThreadsPerGroup + t;
+        lb[(e / TN) * kPitchB + e % TN] = eb[i];
+      }
+    }
+    __syncthreads();
+    if (k0 + 16 < K) load(k0 + 16);
+    if (active) {
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) {
+        float a[kMT], b[kNT];
+#pragma unroll
+        for (int mt = 0; mt < kMT; ++mt) a[mt] = la[(2 * kk + h) * kPitchA + (wm * kMT + mt) * 32 + r];
+#pragma unroll
+        for (int nt = 0; nt < kNT; ++nt) b[nt] = lb[(2 * kk + h) * kPitchB + (wn * kNT + nt) * 32 + r];
+#pragma unroll
+        for (int mt = 0; mt < kMT; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < kNT; ++nt)
+            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
+      }
+    }
+  }
+}
+
+// A thread's share of the largest magnitude among A[0, count) and the K rows of TN columns at B.
+template <int TM, int TN, int kThreadsPerBlock>
+__device__ inline float panel_max(const float* __restrict__ A, size_t count, const float* __restrict__ B, int N, int K,
+                                  int tid) {
+  constexpr int kIn = 8;  // 16-byte loads in flight; the last ones re-read the end
+  float big = 0.0f;
+  auto take = [&](const float* p) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4_any*>(p); };
+  auto fold = [&](dc::f32x4 x) __attribute__((always_inline)) {
+    const float lo = __builtin_fmaxf(__builtin_fabsf(x.x), __builtin_fabsf(x.y));
+    big = __builtin_fmaxf(big, __builtin_fmaxf(lo, __builtin_fmaxf(__builtin_fabsf(x.z), __builtin_fabsf(x.w))));
+  };
+#pragma unroll 1
+  for (size_t i = 4 * tid; i < count; i += 4 * kIn * kThreadsPerBlock) {
+    dc::f32x4 x[kIn];
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) x[u] = take(A + min(i + 4 * u * kThreadsPerBlock, count - 4));
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) fold(x[u]);
+  }
+  constexpr int kRows = 4 * kThreadsPerBlock / TN;
+  B += 4 * (tid % (TN / 4));
+#pragma unroll 1
+  for (int k = tid / (TN / 4); k < K; k += kIn * kRows) {
+    dc::f32x4 x[kIn];
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) x[u] = take(B + (size_t)min(k + u * kRows, K - 1) * N);
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) fold(x[u]);
+  }
+  return big;
+}
+
+template <int TM, int TN>
+struct SplitSmem {
+  unsigned short a[2][3][TM * 16];
+  unsigned short b[2][3][16][TN];
+};
+
+template <int TM, int TN, int WM, int WN, int KS, int D>
+__global__ __launch_bounds__(64 * WM * WN * KS, (TM == 128 && KS == 1 ? 3 : 1)) void gemm_f32_split_kernel(
+    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N, int K, int tiles_m,
+    int tiles_n) {
+  constexpr int kWaves = WM * WN, kT = 64 * kWaves;
+  constexpr int kMT = TM / WM / 32, kNT = TN / WN / 32;      // MFMA tiles per wave
+  constexpr int kBK = 16;
+  constexpr int kA = TM * 4 / kT, kB = TN * 4 / kT;  // quads per thread and k tile
+  using Smem = SplitSmem<TM, TN>;
+  __shared__ __align__(16) Smem sms[KS];
+  __shared__ int s_redo, s_tiny;
+  __shared__ uint32_t s_big;
+  const TileCoord tc = map_tile(tiles_m, tiles_n);
+  const int m0 = tc.tm * TM;
+  const int n0 = min(tc.tn * TN, N - TN);  // the last tile ends at N (N >= TN, by the host)
+  const int tid = threadIdx.x, lane = tid & 63, gwave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = gwave / kWaves, wave = gwave % kWaves, t = tid % kT;
+  Smem& sm = sms[group];
+  const int wm = wave / WN, wn = wave % WN;
+  const int r = lane & 31, h = lane >> 5;
+  const int kt_count = ((K + kBK - 1) / kBK + KS - 1) / KS;  // k tiles per group
+  auto bswz = [](int k) __attribute__((always_inline)) { return TN == 64 ? (k >> 1) & 1 : k & 3; };
+
+  // ---- load side: the lane's element offsets from the tile's first (uniform) A and B element
+  uint32_t ga[kA], gb[kB], wa[kA], wb[kB];  // wa, wb: LDS elements (buffer and plane 0)
+#pragma unroll
+  for (int i = 0; i < kA; ++i) {
+    const int idx = i * kT + t, row = idx / 4, q = idx % 4;
+    ga[i] = (uint32_t)(min(row, M - 1 - m0) * K + 4 * q);
+    wa[i] = (uint32_t)(row * 16 + 8 * ((q >> 1) ^ ((row >> 3) & 1)) + 4 * (q & 1));
+  }
+#pragma unroll
+  for (int i = 0; i < kB; ++i) {
+    const int idx = i * kT + t, krow = idx / (TN / 4), nq = idx % (TN / 4);
+    gb[i] = (uint32_t)(krow * N + 4 * nq);
+    wb[i] = (uint32_t)(krow * TN + 32 * ((nq >> 3) ^ bswz(krow)) + 4 * (nq & 7));
+  }
+  dc::f32x4 sa[D][kA], sb[D][kB];  // D tiles of elements in flight
+  uint32_t tiny = 0xFFFFFFFFu;     // over the lane's elements: see split_quad
+  // The group's k tile KT, every element of which exists.
+  auto load_tile = [&](int KT, dc::f32x4 (&qa)[kA], dc::f32x4 (&qb)[kB]) __attribute__((always_inline)) {
+    const int k0 = (KT * KS + group) * kBK;
+    const float *at = A + (size_t)m0 * K + k0, *bt = B + (size_t)k0 * N + n0;
+#pragma unroll
+    for (int i = 0; i < kA; ++i) qa[i] = *reinterpret_cast<const f32x4_any*>(at + ga[i]);
+#pragma unroll
+    for (int i = 0; i < kB; ++i) qb[i] = *reinterpret_cast<const f32x4_any*>(bt + gb[i]);
+  };
+  // The group's k tile KT, zeros where it lies past K.
+  auto load_checked = [&](int KT, dc::f32x4 (&qa)[kA], dc::f32x4 (&qb)[kB]) __attribute__((always_inline)) {
+    const int k0 = (KT * KS + group) * kBK;
+    const int klim = K - k0;  // k rows of the tile that exist (16 or more: all; none: the tile is zero)
+    const float *at = A + (size_t)m0 * K + k0, *bt = B + (size_t)k0 * N + n0;
+#pragma unroll
+    for (int i = 0; i < kA; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qa[i][e] = 4 * ((i * kT + t) % 4) + e < klim ? at[ga[i] + e] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < kB; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qb[i][e] = (i * kT + t) / (TN / 4) < klim ? bt[gb[i] + e] : 0.0f;
+  };
+  auto split_tile = [&](auto BUF, const dc::f32x4 (&qa)[kA], const dc::f32x4 (&qb)[kB]) __attribute__((always_inline)) {
+    constexpr int kBuf = decltype(BUF)::value;
+    u32x2 piece[3];
+#pragma unroll
+    for (int i = 0; i < kA; ++i) {
+      split_quad(qa[i], piece, &tiny);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(&sm.a[kBuf][p][0] + wa[i]) = piece[p];
+    }
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+      split_quad(qb[i], piece, &tiny);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(&sm.b[kBuf][p][0][0] + wb[i]) = piece[p];
+    }
+  };
+
+  // ---- read side
+  const unsigned char* lds = reinterpret_cast<const unsigned char*>(&sm);
+  const uint32_t aoff = (uint32_t)((wm * 32 * kMT + r) * 32 + 16 * (h ^ ((r >> 3) & 1)));
+  uint32_t boff[kNT];
+  {
+    const int j = (lane & 15) >> 2, p4 = lane & 3, cg = (lane >> 4) & 1;
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt)
+      boff[nt] = (uint32_t)offsetof(Smem, b) + (uint32_t)((8 * h + j) * 2 * TN) +
+                 64u * (uint32_t)((kNT * wn + nt) ^ bswz(j)) + (uint32_t)(32 * cg + 8 * p4);
+  }
+  f32x16 acc[kMT][kNT];
+#pragma unroll
+  for (int i = 0; i < kMT; ++i)
+#pragma unroll
+    for (int j = 0; j < kNT; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+  auto read_a = [&](int buf, int p, bf16x8 (&a)[kMT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int mt = 0; mt < kMT; ++mt)
+      a[mt] = __builtin_bit_cast(
+          bf16x8, *reinterpret_cast<const u16x8*>(lds + aoff + ((buf * 3 + p) * TM + mt * 32) * 32));
+  };
+  auto read_b = [&](int buf, int p, bf16x8 (&b)[kNT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt) {
+      const unsigned char* q = lds + boff[nt] + (buf * 3 + p) * 16 * 2 * TN;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(q));
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(q + 4 * 2 * TN));
+      b[nt] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+  };
+  auto mfmas = [&](const bf16x8 (&a)[kMT], const bf16x8 (&b)[kNT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int mt = 0; mt < kMT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < kNT; ++nt)
+        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
+  };
+  // Fragments: plane 0 of B twice (the next tile's is read while this one's is still in use).
+  bf16x8 a0[kMT], a1[kMT], a2[kMT], b0[2][kNT], b1[kNT], b2[kNT];
+  constexpr int kMfmas = 3 * kMT * kNT, kSplits = kA + kB;
+  // One k tile (buffer BUF) in two regions of three products each (small ones first), the barrier
+  // between them. First region: the reads of the planes that come last, and the split of the next tile
+  // (elements qa, qb) into the other buffer between the products. Second region: the reads of the
+  // next tile's first fragments between the products, so none of the LDS time is exposed.
+  auto first = [&](auto BUF, const dc::f32x4 (&qa)[kA], const dc::f32x4 (&qb)[kB]) __attribute__((always_inline)) {
+    constexpr int kBuf = decltype(BUF)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(kBuf, 0, a0);
+    read_b(kBuf, 2, b2);
+    split_tile(std::integral_constant<int, 1 - kBuf>{}, qa, qb);
+    mfmas(a2, b0[kBuf]);
+    mfmas(a1, b1);
+    mfmas(a1, b0[kBuf]);
+    __builtin_amdgcn_sched_group_barrier(0x100, kMT + 2 * kNT, 0);
+#pragma unroll
+    for (int i = 0; i < kMfmas; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, (26 * kSplits + kMfmas - 1) / kMfmas, 0);
+      __builtin_amdgcn_sched_group_barrier(0x200, (3 * kSplits + kMfmas - 1) / kMfmas, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto second = [&](auto BUF) __attribute__((always_inline)) {
+    constexpr int kBuf = decltype(BUF)::value, kNext = 1 - kBuf;
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(kNext, 2, a2);
+    read_b(kNext, 0, b0[kNext]);
+    read_a(kNext, 1, a1);
+    mfmas(a0, b2);
+    mfmas(a0, b1);
+    mfmas(a0, b0[kBuf]);
+    read_b(kNext, 1, b1);
+#pragma unroll
+    for (int i = 0; i < 2 * kMT * kNT; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x100, (2 * kMT + 2 * kNT + 2 * kMT * kNT - 1) / (2 * kMT * kNT), 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (tid == 0) s_redo = s_tiny = s_big = 0;
+  constexpr uint32_t kTinyBits = 2u * __builtin_bit_cast(uint32_t, kSplitMin) - 1u;
+  constexpr std::integral_constant<int, 0> kBuf0{};
+  constexpr std::integral_constant<int, 1> kBuf1{};
+  static_assert(D == 1 || D == 2, "the loop is unrolled by two");
+  // The group's last tile, the only one that can lie past K, comes first (checked loads); then tiles
+  // 0, 1, ...: step p > 0 is tile p - 1. The host sees to kt_count >= 2. Loads past the last step
+  // re-read its tile (unused): no branch in the loop, so its waits for memory cover just the tile
+  // that is split next.
+  load_checked(kt_count - 1, sa[0], sb[0]);
+  split_tile(kBuf0, sa[0], sb[0]);
+  __syncthreads();  // s_redo, s_tiny, s_big are set
+  {  // nothing but small values in a wave's share of the first tile: they are no exception here
+    float big_a = 0.0f, big_b = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4 * kA; ++i) big_a = __builtin_fmaxf(big_a, __builtin_fabsf(sa[0][i / 4][i % 4]));
+#pragma unroll
+    for (int i = 0; i < 4 * kB; ++i) big_b = __builtin_fmaxf(big_b, __builtin_fabsf(sb[0][i / 4][i % 4]));
+    const bool small_a = __any(big_a > 0.0f) && !__any(big_a >= kSplitMin);
+    const bool small_b = __any(big_b > 0.0f) && !__any(big_b >= kSplitMin);
+    if (small_a || small_b) s_redo = 1;
+  }
+  for_each_index([&](auto I) __attribute__((always_inline)) {
+    load_tile(min(I.value, kt_count - 2), sa[(1 + I.value) % D], sb[(1 + I.value) % D]);
+  }, std::make_integer_sequence<int, D>{});
+  __syncthreads();
+  read_a(0, 2, a2);
+  read_b(0, 0, b0[0]);
+  read_a(0, 1, a1);
+  read_b(0, 1, b1);
+  // Step p in buffer I = p % 2: its products and the split of step p + 1, whose element set then
+  // takes step p + 1 + D.
+  auto one = [&](int p, auto I) __attribute__((always_inline)) {
+    constexpr int i = decltype(I)::value, set = (i + 1) % D;
+    first(I, sa[set], sb[set]);
+    __syncthreads();
+    load_tile(min(p + D, kt_count - 2), sa[set], sb[set]);
+    second(I);
+  };
+  const bool early = __builtin_amdgcn_readfirstlane(s_redo) != 0;
+  __builtin_assume(kt_count > 1);
+  int p = 0;
+  do {
+    if (early) break;
+    one(p, kBuf0);
+    if (p + 1 >= kt_count) break;
+    one(p + 1, kBuf1);
+    p += 2;
+  } while (p < kt_count);
+  if (tiny < kTinyBits) s_tiny = 1;
+
+  if constexpr (KS > 1) {  // the groups' sums, added in group order by group 0
+    constexpr int kSums = kT * kMT * kNT * 16;
+    static_assert(sizeof(sms) >= (KS - 1) * kSums * sizeof(float), "the groups' sums fit in the buffers");
+    float* part = reinterpret_cast<float*>(&sms[0]) + (group - 1) * kSums + t;
+    __syncthreads();
+    if (group > 0)
+#pragma unroll
+      for (int i = 0; i < kMT * kNT * 16; ++i) part[i * kT] = acc[i / 16 / kNT][i / 16 % kNT][i % 16];
+    __syncthreads();
+    if (group == 0)
+#pragma unroll
+      for (int g = 1; g < KS; ++g) {
+        const float* other = reinterpret_cast<const float*>(&sms[0]) + (g - 1) * kSums + t;
+#pragma unroll
+        for (int i = 0; i < kMT * kNT * 16; ++i) acc[i / 16 / kNT][i / 16 % kNT][i % 16] += other[i * kT];
+      }
+  }
+  __syncthreads();
+  float least = 0.0f;  // sums below this may have lost more than 2^-26 of themselves to small values
+  if (s_tiny && !early) {  // uniform
+    const float big = panel_max<TM, TN, kT * KS>(A + (size_t)m0 * K, (size_t)min(TM, M - m0) * K, B + n0, N, K, tid);
+    atomicMax(&s_big, __builtin_bit_cast(uint32_t, big));
+    __syncthreads();
+    least = __builtin_bit_cast(float, s_big) * (float)K * 0x1p-107f;  // 2 K lost pieces of at most 2^-134
+  }
+  if (group == 0) {
+    float z = 0.0f;  // stays zero where every sum is finite (x - x is not otherwise)
+    bool low = false;
+#pragma unroll
+    for (int i = 0; i < kMT * kNT * 16; ++i) {
+      const float x = acc[i / 16 / kNT][i / 16 % kNT][i % 16];
+      z += x - x;
+      low |= __builtin_fabsf(x) < least;
+    }
+    if (!(z == 0.0f) || low) s_redo = 1;
+  }
+  __syncthreads();
+  if (s_redo) {
+    static_assert(sizeof(Smem) >= 16 * (TM + TN + 64) * sizeof(float), "the fp32 staging fits in the buffers");
+    float* la = reinterpret_cast<float*>(&sms[0]);
+    f32_tile_direct<TM, TN, kMT, kNT, kT>(A, B, M, N, K, m0, n0, t, group == 0, wm, wn, la, la + 16 * (TM + 32), acc);
+  }
+  if (group > 0) return;
+  // acc[mt][nt][v] holds C[row][col], row = 8*(v/4) + 4*h + v%4, col = r (within the 32×32 tile).
+  // Only the columns of this tile's own place are stored.
+  const bool whole = m0 + TM <= M && n0 + TN <= N && n0 == tc.tn * TN;
+#pragma unroll
+  for (int mt = 0; mt < kMT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt) {
+      const int col = n0 + (wn * kNT + nt) * 32 + r;
+      const bool cok = col < N && col >= tc.tn * TN;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int row = m0 + (wm * kMT + mt) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+        if (whole || (cok && row < M)) C[(size_t)row * N + col] = acc[mt][nt][v];
+      }
+    }
+}
+
 // Round-to-nearest-even fp32 -> bf16 (quiet NaN kept NaN).
 __global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float* __restrict__ x, unsigned short* __restrict__ y,
                                                           int64_t n) {
@@ -743,6 +1186,21 @@ void launch_bf16(dc_hip_ctx* ctx, const unsigned short* a, const unsigned short*
       a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
 }
 
+// The split kernel where its conditions hold (a whole tile of columns, two k tiles per group, and 32-bit
+// element offsets within a panel), else the checked fp32 kernel.
+template <int TM, int TN, int WM, int WN, int KS, int D>
+void launch_f32(dc_hip_ctx* ctx, const float* a, const float* b, float* c, int64_t m, int64_t n, int64_t k) {
+  if (n >= TN && k > 16 * KS && TM * k < INT32_MAX && 16 * n < INT32_MAX) {
+    const int tiles_m = (int)((m + TM - 1) / TM), tiles_n = (int)((n + TN - 1) / TN);
+    gemm_f32_split_kernel<TM, TN, WM, WN, KS, D><<<(unsigned)(tiles_m * tiles_n), 64 * WM * WN * KS, 0, ctx->stream>>>(
+        a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
+  } else {
+    const int tiles_m = (int)((m + 63) / 64), tiles_n = (int)((n + 63) / 64);
+    gemm_f32_kernel<kBKf32, true, 64><<<(unsigned)(tiles_m * tiles_n), kThreads, 0, ctx->stream>>>(
+        a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
+  }
+}
+
 int32_t check_dims(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n < 0 || k < 0) return DC_ERR_INVALID_ARGUMENT;
   if (m > INT32_MAX / 2 || n > INT32_MAX / 2 || k > INT32_MAX / 2) return DC_ERR_INVALID_ARGUMENT;
@@ -760,27 +1218,33 @@ DC_HIP_API int32_t dc_hip_gemm_f32(dc_hip_ctx* ctx, const float* a, const float*
   if (!c || (k > 0 && (!a || !b))) return DC_ERR_INVALID_ARGUMENT;
   DC_CTX_ENTER(ctx);
   if (k == 0) return dc::zero_async(ctx, c, (size_t)(m * n) * sizeof(float));
-  // 128×128 tiles unless that leaves fewer than two per CU; then 64×64 (four times the tiles)
-  const int64_t tiles128 = ((m + 127) / 128) * ((n + 127) / 128);
-  const bool small = tiles128 < 2 * (int64_t)std::max(1, ctx->cu_count);
-  const int T = small ? 64 : 128;
-  const int tiles_m = (int)((m + T - 1) / T), tiles_n = (int)((n + T - 1) / T);
-  const unsigned grid = (unsigned)(tiles_m * tiles_n);
-  // full tiles take the direct-to-LDS kernel; its A panel (T rows of k floats) is one buffer range
-  const bool full = (m % T == 0) && (n % T == 0) && (k % kBKd == 0) && dc::aligned16(a) && dc::aligned16(b) &&
-                    (int64_t)T * k * 4 < ((int64_t)1 << 31) && ((int64_t)kBKd * n + T) * 4 < ((int64_t)1 << 31);
-#define DC_GEMM_F32_DMA(TT) \
-  gemm_f32_dma_kernel<TT><<<grid, kThreads, 0, ctx->stream>>>(a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n)
-#define DC_GEMM_F32_CHECKED(TT)                                                                                 \
-  gemm_f32_kernel<kBKf32, true, TT><<<grid, kThreads, 0, ctx->stream>>>(a, b, c, (int)m, (int)n, (int)k, tiles_m, \
-                                                                       tiles_n)
-  if (small) {
-    if (full) DC_GEMM_F32_DMA(64); else DC_GEMM_F32_CHECKED(64);
+  // The widest tile that still gives the chip enough workgroups, then a k dimension split over the
+  // wave groups of a workgroup. Measured (us; "xG": G groups; "f32": the fp32 instructions, direct-to-LDS):
+  //   8192^3: 256 4504, 128 5285, f32 7312;  4096^3: 561 / 658 / 925;  3500^3: 422 / 561, x2 572
+  //   3072x3072x1024 (144 tiles of 256, 576 of 128): 117 / 115, x2 134, f32 138
+  //   2048^3 (256 of 128): 218 / 104, x2 90.5, 64 118;  1536^3 (144 of 128): 167 / 76, x2 59, 64 64
+  //   1279x1281x641 (441 of 64): 128x2 29, 64 22.7, x2 20.8, x4 24.7
+  //   1023^3 (256 of 64): 25, x2 19.3, x4 19.5;  300x300x8000 (25 of 64): 164, x2 113, x4 99
+  //   full 64-tiles, f32 / best split: 256^3 6.2 / 8.8, 512^3 10.3 / 12, 1024^3 19.7 / 19.9,
+  //   512x512x4096 66 / 53: few tiles of a short k leave the split's longer start-up uncovered
+  const int64_t cus = std::max(1, ctx->cu_count);
+  auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
+  if (m % 64 == 0 && n % 64 == 0 && k % kBKd == 0 && dc::aligned16(a) && dc::aligned16(b) && tiles(64) <= cus && k <= 1024) {
+    // (each buffer range of the kernel, 64 rows of k floats or 32 rows of n, is below 2 GiB by then)
+    const int tiles_m = (int)(m / 64), tiles_n = (int)(n / 64);
+    gemm_f32_dma_kernel<64><<<(unsigned)(tiles_m * tiles_n), kThreads, 0, ctx->stream>>>(a, b, c, (int)m, (int)n, (int)k,
+                                                                                       tiles_m, tiles_n);
+  } else if (n >= 256 && 2 * tiles(256) > cus) {
+    launch_f32<256, 256, 2, 4, 1, 1>(ctx, a, b, c, m, n, k);
+  } else if (n >= 128 && tiles(128) > cus) {
+    launch_f32<128, 128, 2, 2, 1, 1>(ctx, a, b, c, m, n, k);
+  } else if (n >= 128 && 2 * tiles(128) > cus && k >= 256) {
+    launch_f32<128, 128, 2, 2, 2, 2>(ctx, a, b, c, m, n, k);
+  } else if (tiles(64) > cus || k < 1536) {
+    launch_f32<64, 64, 2, 2, 2, 2>(ctx, a, b, c, m, n, k);
   } else {
-    if (full) DC_GEMM_F32_DMA(128); else DC_GEMM_F32_CHECKED(128);
+    launch_f32<64, 64, 2, 2, 4, 2>(ctx, a, b, c, m, n, k);
   }
-#undef DC_GEMM_F32_DMA
-#undef DC_GEMM_F32_CHECKED
   return dc::last_launch_status();
 }
 

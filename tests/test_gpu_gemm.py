@@ -192,3 +192,50 @@ def test_gemm_bf16_ragged_tiles(ctx, shape):
     a[1:] = np.inf
     c0 = run_gemm(ctx, a, b, kind="bf16")[0]
     assert np.array_equal(c0, c[0])
+
+
+# One shape per tile choice of the fp32 dispatch (on 256 CUs), rows, columns and last k tile ragged:
+# 256-tiles, 128-tiles with one and two k groups, 64-tiles with two and four; the smallest k that
+# the two- and four-group kernels take, and one less.
+@pytest.mark.parametrize("shape", [(2824, 3083, 50), (2200, 2057, 131), (1799, 1911, 257), (300, 333, 61),
+                                   (129, 131, 1537), (65, 64, 33), (65, 64, 32), (200, 1000, 49)])
+def test_gemm_f32_split_tiles(ctx, shape):
+    m, n, k = shape
+    a, b = make_inputs(m, n, k)
+
+    def check(a, b):
+        c = run_gemm(ctx, a, b)
+        a64, b64 = a.astype(np.float64), b.astype(np.float64)
+        # each product within 2^-24 of itself, k additions each within one float32 ulp
+        assert np.all(np.abs(c - a64 @ b64) <= (k + 1) * 2.0 ** -23 * (np.abs(a64) @ np.abs(b64)))
+        return c
+
+    c = check(a, b)
+    # values whose bf16 pieces would not hold them: everywhere, and in one row
+    check(a * np.float32(2.0 ** -110), b)
+    tiny = a.copy()
+    tiny[m // 2] *= np.float32(2.0 ** -120)
+    c2 = check(tiny, b)
+    far = np.abs(np.arange(m) - m // 2) > 256  # rows of other tiles: the very same sums
+    assert np.array_equal(c2[far], c[far])
+    check(np.where(np.arange(m * k).reshape(m, k) % 3 == 0, a * np.float32(2.0 ** -115), a), b)
+    # infinities, NaN and values that round to infinity in bf16 stay in their rows
+    odd = a.copy()
+    odd[0, 0], odd[1, 1], odd[2, k - 1], odd[3, 0] = np.inf, np.nan, -np.inf, 3.4e38
+    bz = b.copy()
+    bz[0, 0] = 0.0
+    got = run_gemm(ctx, odd, bz)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = (odd.astype(np.float64) @ bz.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(np.isnan(got[:3]), np.isnan(ref[:3])) and np.array_equal(np.isinf(got[:3]), np.isinf(ref[:3]))
+    # (row 3 by the bound above: its column 0 is an ordinary sum that cancels, no relative bound holds)
+    bound3 = (k + 1) * 2.0 ** -23 * (np.abs(odd[3]).astype(np.float64) @ np.abs(bz).astype(np.float64))
+    assert np.isfinite(got[3:]).all() and np.all(np.abs(got[3] - ref[3].astype(np.float64)) <= bound3)
+
+
+def test_gemm_f32_split_permutation_exact(ctx):
+    n = 2100  # one nonzero term per entry: the three pieces add up to the value itself
+    a, _ = make_inputs(n, n, n)
+    perm = np.eye(n, dtype=np.float32)[np.random.default_rng(1).permutation(n)]
+    assert np.array_equal(run_gemm(ctx, perm, a), perm @ a)
+    assert np.array_equal(run_gemm(ctx, a, perm), a @ perm)
