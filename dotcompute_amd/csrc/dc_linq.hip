@@ -1,7 +1,8 @@
 // dc_linq.hip — fused LINQ Where/Select(/Sum) kernels for gfx950.
 //
-// One prebuilt kernel per terminal (ToArray, Sum) interprets the register program that the host
-// fusion planner builds from the chain's lambdas (dc_linq_chain, program model in
+// One prebuilt kernel per terminal (ToArray, Sum) and form of program (one- and two-stage affine
+// chains, longer affine chains, a comparison pair and a short polynomial, anything else: interpreted)
+// runs the register program that the host fusion planner builds from the chain's lambdas (dc_linq_chain, program model in
 // include/dotcompute_hip.h). The program lives in the kernel arguments, so every instruction is
 // wave-uniform: dispatch is scalar branching, and each instruction is applied to the 16 elements a
 // thread holds in registers.
@@ -212,6 +213,82 @@ inline bool lower_canon2(const AffineChain& ch, int* shape, int* cmp, RdConst* o
   return true;
 }
 
+// Lowers `Where(y <cmp> c [&&/|| y <cmp> c']).Select(steps)` (PolyChain; either part optional) of a
+// validated program; false when the program has another form. *has_rem: y = x % constant (int32).
+inline bool lower_poly(const dc_linq_chain& prog, bool is_int, PolyChain* out, bool* has_rem) {
+  PolyChain p{};
+  *has_rem = false;
+  auto bits = [](const dc_linq_instr& in) { return __builtin_bit_cast(uint32_t, in.imm_i32); };
+  for (int k = 0; k < 2; ++k) p.inv[k] = ~0u;  // no comparison: true
+  int pc = 0;
+  auto at = [&](int i) { return i < prog.n_instr ? prog.code[i] : dc_linq_instr{}; };
+  auto is_load = [&](int i) { return i < prog.n_instr && at(i).op == DC_LQ_LOAD && at(i).src == DC_LQ_SRC_ELEM; };
+  auto is_cmp = [&](int i) { return at(i).op >= DC_LQ_CMP_GT && at(i).op <= DC_LQ_CMP_NE && at(i).src == DC_LQ_SRC_IMM; };
+  auto compare = [&](int k, const dc_linq_instr& in) {
+    // int32: a "less" is the complement of its opposite; float (NaN fails both): of the negated operands
+    const bool less = in.op == DC_LQ_CMP_LT || in.op == DC_LQ_CMP_LE;
+    const bool equality = in.op == DC_LQ_CMP_EQ || in.op == DC_LQ_CMP_NE;
+    p.flip[k] = less && !is_int ? 0x80000000u : 0u;
+    p.t[k] = bits(in) ^ p.flip[k];
+    const bool ge = equality || in.op == DC_LQ_CMP_GE || in.op == (is_int ? DC_LQ_CMP_LT : DC_LQ_CMP_LE);
+    const bool gt = equality || in.op == DC_LQ_CMP_GT || in.op == (is_int ? DC_LQ_CMP_LE : DC_LQ_CMP_LT);
+    p.ge[k] = ge ? ~0u : 0u;
+    p.gt[k] = gt ? ~0u : 0u;
+    p.inv[k] = in.op == DC_LQ_CMP_NE || (less && is_int) ? ~0u : 0u;
+  };
+  if (!is_load(pc)) return false;
+  int q = pc + 1;
+  if (is_int && at(q).op == DC_LQ_REM && at(q).src == DC_LQ_SRC_IMM && at(q).imm_i32 != 0 && at(q).imm_i32 != 1 &&
+      at(q).imm_i32 != -1) {
+    const dc::DivMagic g = dc::div_magic(at(q).imm_i32);
+    p.rem_m = g.m;
+    p.rem_s = g.s;
+    p.rem_d = g.d;
+    *has_rem = true;
+    ++q;
+  }
+  bool any = false;
+  if (is_cmp(q) && at(q).mode == DC_LQ_CMP_SET) {
+    compare(0, at(q++));
+    if (is_cmp(q) && at(q).mode != DC_LQ_CMP_SET) {
+      const bool either = at(q).mode == DC_LQ_CMP_OR;
+      compare(1, at(q++));
+      if (either) {
+        p.inv[0] = ~p.inv[0];
+        p.inv[1] = ~p.inv[1];
+        p.inv_both = ~0u;
+      }
+    }
+    if (at(q).op != DC_LQ_FILTER || q >= prog.n_instr) return false;
+    pc = q + 1;
+    any = true;
+  } else if (*has_rem) {
+    return false;
+  }
+  if (is_load(pc)) {
+    q = pc + 1;
+    int k = 0;
+    for (; q < prog.n_instr && at(q).op != DC_LQ_MAP; ++q, ++k) {
+      const dc_linq_instr in = at(q);
+      if (k == 3 || (in.op != DC_LQ_ADD && in.op != DC_LQ_SUB && in.op != DC_LQ_MUL) ||
+          (in.src != DC_LQ_SRC_IMM && in.src != DC_LQ_SRC_ELEM))
+        return false;
+      p.use[k] = ~0u;
+      p.mul[k] = in.op == DC_LQ_MUL ? ~0u : 0u;
+      p.elem[k] = in.src == DC_LQ_SRC_ELEM ? ~0u : 0u;
+      p.neg[k] = in.op == DC_LQ_SUB && p.elem[k] ? ~0u : 0u;
+      // v - c is v + (-c): exact for floats, wrapping for ints
+      p.c[k] = in.op != DC_LQ_SUB ? bits(in) : is_int ? 0u - bits(in) : bits(in) ^ 0x80000000u;
+    }
+    if (q >= prog.n_instr) return false;
+    pc = q + 1;
+    any = true;
+  }
+  if (!any || pc != prog.n_instr) return false;
+  *out = p;
+  return true;
+}
+
 struct ReducePlan {
   int mode;
   AffineChain aff;
@@ -230,10 +307,20 @@ inline ReducePlan reduce_plan(const dc_linq_chain& prog) {
   ReducePlan p{};
   p.k = RdConst{0.0f, 1.0f, -0.0f};
   int shape = 0, cmp = DC_LQ_CMP_GT;
+  bool rem = false;
   if (!lower_affine(prog, &p.aff))
-    p.mode = program_uses_libm(prog) ? kRdInterpLibm : program_uses_saves(prog) ? kRdInterpSaves : kRdInterp;
+    p.mode = lower_poly(prog, false, &p.aff.poly, &rem) ? kRdPolyF32 : program_uses_libm(prog) ? kRdInterpLibm : program_uses_saves(prog) ? kRdInterpSaves : kRdInterp;
   else if (lower_canon2(p.aff, &shape, &cmp, &p.k)) p.mode = rd_canon(shape, cmp);
   else p.mode = kRdAffine;
+  return p;
+}
+
+// The round-robin ToArray's plan of an int32 program: the comparison-and-polynomial form, else the
+// interpreter.
+inline ReducePlan to_array_plan_i32(const dc_linq_chain& prog) {
+  ReducePlan p = reduce_plan_i32(prog);
+  bool rem = false;
+  if (lower_poly(prog, true, &p.aff.poly, &rem)) p.mode = rem ? kRdPolyRemI32 : kRdPolyI32;
   return p;
 }
 
@@ -251,6 +338,7 @@ void rd_dispatch(int mode, F&& f) {
     DC_RD_CASE(kRdInterpSaves)
     DC_RD_CASE(kRdInterpLibm)
     DC_RD_CASE(kRdAffine)
+    DC_RD_CASE(kRdPolyF32)
     DC_RD_CASE(rd_canon(kShapeM, DC_LQ_CMP_GT))
     DC_RD_CMP_MODES(DC_RD_CASE, kShapeF)
     DC_RD_CMP_MODES(DC_RD_CASE, kShapeFM)
@@ -1266,6 +1354,8 @@ const void* rounds_kernel(int mode) {
   const void* fn = nullptr;
   auto pick = [&](auto m) { fn = reinterpret_cast<const void*>(&where_select_rounds_kernel<decltype(m)::value>); };
   if (rd_is_int(mode)) rd_dispatch_i32(mode, pick);
+  else if (mode == kRdPolyI32) pick(std::integral_constant<int, kRdPolyI32>{});
+  else if (mode == kRdPolyRemI32) pick(std::integral_constant<int, kRdPolyRemI32>{});
   else rd_dispatch(mode, pick);
   return fn;
 }
@@ -1273,7 +1363,7 @@ const void* rounds_kernel(int mode) {
 // Every program variant (rd_dispatch's and rd_dispatch_i32's cases).
 std::vector<int> all_reduce_modes() {
   std::vector<int> m = {kRdInterp, kRdInterpSaves, kRdInterpLibm, kRdAffine, kRdInterpI32, kRdInterpI32Saves,
-                        rd_canon(kShapeM, DC_LQ_CMP_GT)};
+                        kRdPolyF32, kRdPolyI32, kRdPolyRemI32, rd_canon(kShapeM, DC_LQ_CMP_GT)};
   for (int shape : {kShapeF, kShapeFM, kShapeMF})
     for (int cmp = DC_LQ_CMP_GT; cmp <= DC_LQ_CMP_NE; ++cmp) m.push_back(rd_canon(shape, cmp));
   return m;
@@ -1354,13 +1444,13 @@ int32_t launch_to_array(dc_hip_ctx* ctx, const dc_linq_chain* chain, bool is_int
                         float* output, int64_t* count_out) {
   uint64_t* fault_word = reinterpret_cast<uint64_t*>(ctx->counters + DC_SLOT_LINQ_FAULT);
   if ((chain->flags & DC_LINQ_FLAG_ORDERED_GRID) == 0 && use_rounds(ctx, input, n)) {
-    const ReducePlan plan = is_int ? reduce_plan_i32(*chain) : reduce_plan(*chain);
+    const ReducePlan plan = is_int ? to_array_plan_i32(*chain) : reduce_plan(*chain);
     const void* fn = rounds_kernel(plan.mode);
     // Programs the prebuilt kernels interpret can run on a kernel compiled for them
     // (dc::linq_jit_rounds). Switched off: a compiled kernel for a filtered division faulted the
     // device and its cause is not found yet, so every program runs on the interpreter.
     hipFunction_t jit = nullptr;
-    const bool interpreted = is_int || rd_is_float_interp(plan.mode);
+    const bool interpreted = rd_is_int(plan.mode) || rd_is_float_interp(plan.mode);
     if (kLaunchCompiled && interpreted && n >= DC_LINQ_COMPILE_MIN_ELEMENTS &&
         (chain->flags & DC_LINQ_FLAG_INTERPRET) == 0) {
       jit = dc::linq_jit_rounds(ctx, *chain, is_int);

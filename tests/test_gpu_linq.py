@@ -611,3 +611,40 @@ def test_fold_random_programs(ctx, seed):
             assert np.sign(got) == np.sign(ref) and abs(int(g) - int(r)) <= 2, (got, ref)
         elif rcnt:
             assert same_floats(np.array([got]), np.array([ref]))
+
+
+# Comparison-pair-and-polynomial programs (a kernel of their own on the round-robin grid and in the
+# reductions): run_to_array compares that grid with the lookback grid's interpreter bit for bit, and
+# both are compared with the oracle, over zeros of both signs, infinities, NaN, denormals and the
+# thresholds themselves. 7 elements past three tiles; one head element.
+POLY_SECOND = [None, (hip.CMP_AND, CMP_LT, 0.5), (hip.CMP_OR, CMP_LE, -0.5), (hip.CMP_OR, CMP_EQ, 0.25),
+               (hip.CMP_AND, CMP_NE, 0.0)]
+POLY_STEPS = [None, [], [(MUL, SRC_ELEM, 0)], [(MUL, SRC_ELEM, 0), (ADD, SRC_ELEM, 0)],
+              [(SUB, SRC_ELEM, 0), (ADD, SRC_IMM, 3.0), (MUL, SRC_ELEM, 0)], [(SUB, SRC_IMM, 0.1), (MUL, SRC_IMM, -3.0)]]
+
+
+@pytest.mark.parametrize("cmp", [None, CMP_GT, CMP_GE, CMP_LT, CMP_LE, CMP_EQ, CMP_NE])
+@pytest.mark.parametrize("second", range(len(POLY_SECOND)))
+def test_poly_programs_match_interpreter(ctx, cmp, second):
+    if cmp is None and second:
+        pytest.skip("a second comparison needs a first")
+    x = oracle.gen_uniform_f32(3 * RR_TILE + 7, 900 + second, 0)
+    x[::11] = np.resize(np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-40, 0.25, -0.25, 0.5, -0.5], np.float32), x[::11].size)
+    for i, steps in enumerate(POLY_STEPS):
+        code = []
+        if cmp is not None:
+            code += [(LOAD, SRC_ELEM, 0), (cmp, SRC_IMM, 0.25)]
+            if POLY_SECOND[second]:
+                mode, op, imm = POLY_SECOND[second]
+                code.append((op, SRC_IMM, imm, mode))
+            code.append((FILTER, SRC_IMM, 0))
+        if steps is not None:
+            code += [(LOAD, SRC_ELEM, 0)] + steps + [(MAP, SRC_IMM, 0)]
+        if not code:
+            continue
+        prog = LinqChain.assemble(code)
+        assert same_floats(run_to_array(ctx, prog, x, offset=i % 4), oracle.linq_where_select(prog, x))
+        fin = x[np.isfinite(x)]
+        got, cnt = run_sum(ctx, prog, fin)
+        _, sd, rc = oracle.linq_where_select_sum(prog, fin)
+        assert cnt == rc and abs(got - sd) <= 1e-5 * math.log2(fin.size) * max(abs(sd), 1.0)

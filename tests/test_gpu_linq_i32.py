@@ -355,3 +355,24 @@ def test_division_constants_when_the_program_is_full(ctx):
     ref, rf = oracle.linq_where_select_i32(ch, x)
     assert f == rf == -1 and np.array_equal(got, ref)
     assert run_sum(ctx, ch, x) == oracle.linq_where_select_sum_i32(ch, x)
+
+
+# Comparison-pair-and-polynomial programs over int32 (their own round-robin kernels, with and without
+# x % constant): run_to_array compares that grid with the lookback grid's interpreter, and both are
+# compared with the oracle, over the extremes of int and both signs.
+@pytest.mark.parametrize("rem", [None, 2, -3, 7, 1000003, -2147483648])
+@pytest.mark.parametrize("cmp", [hip.CMP_GT, hip.CMP_GE, hip.CMP_LT, hip.CMP_LE, hip.CMP_EQ, hip.CMP_NE])
+def test_poly_programs_match_oracle(ctx, rem, cmp):
+    x = oracle.gen_uniform_i32(20_011, 77, 1, -1000, 1000)
+    x[::13] = np.resize(np.array([0, 1, -1, 2147483647, -2147483648, -2147483647], np.int32), x[::13].size)
+    load, imm, elem = (hip.LOAD, hip.SRC_ELEM, 0), hip.SRC_IMM, hip.SRC_ELEM
+    seconds = [None, (hip.CMP_LT, imm, 500, hip.CMP_AND), (hip.CMP_EQ, imm, -1, hip.CMP_OR),
+               (hip.CMP_LE, imm, -700, hip.CMP_OR)]
+    maps = [[], [(hip.MUL, elem, 0)], [(hip.SUB, elem, 0), (hip.ADD, imm, 5), (hip.MUL, elem, 0)],
+            [(hip.MUL, imm, -2147483648), (hip.SUB, imm, -2147483648)]]
+    for i, (second, steps) in enumerate((s, m) for s in seconds for m in maps):
+        code = [load] + ([(hip.REM, imm, rem)] if rem else []) + [(cmp, imm, 0)] + ([second] if second else [])
+        code += [(hip.FILTER, 0, 0)] + ([load] + steps + [(hip.MAP, 0, 0)] if steps else [])
+        ch = hip.LinqChain.assemble(code, int32=True)
+        got = run_to_array(ctx, ch, x, offset=i % 4)[0]
+        assert np.array_equal(got, oracle.linq_where_select_i32(ch, x)[0])
