@@ -193,6 +193,25 @@ def test_spmv_int_wraps_like_csharp(ctx, rows):
     assert np.array_equal(y, ref)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32])
+def test_spmv_row_lengths_around_the_batched_reads(ctx, dtype):
+    """Rows are summed in batches of LDS reads: every length up to two batches of 16 and past, around
+    the wave size, and around the long-row threshold (512) gives the sequential loop's bits."""
+    lengths = np.array(list(range(42)) + [63, 64, 65, 255, 256, 257] + list(range(500, 513)) + [0, 1, 513, 2], np.int64)
+    rp = np.concatenate([[0], np.cumsum(np.concatenate([lengths, lengths[::-1]]))]).astype(np.int32)
+    nnz, cols = int(rp[-1]), 1000
+    col = oracle.gen_uniform_i32(nnz, 71, 0, 0, cols - 1)
+    if dtype == np.int32:
+        val, x = oracle.gen_uniform_i32(nnz, 72, 1, -2_000_000_000, 2_000_000_000), oracle.gen_uniform_i32(cols, 73, 2, -70_000, 70_000)
+        ref = oracle.spmv_csr_i32(rp, col, val, x)
+    else:
+        val, x = oracle.gen_uniform_f32(nnz, 72, 1).astype(dtype), oracle.gen_uniform_f32(cols, 73, 2).astype(dtype)
+        ref = (oracle.spmv_csr_f32 if dtype == np.float32 else oracle.spmv_csr_f64d)(rp, col, val, x)
+    y = spmv_gpu_typed(ctx, rp, col, val, x)
+    short = np.diff(rp) <= 512
+    assert y[short].tobytes() == ref[short].tobytes()
+
+
 def test_spmv_typed_dimension_check(ctx):
     rp = np.array([0, 1], np.int32)
     col = np.array([0], np.int32)
