@@ -57,17 +57,17 @@ __device__ inline int32_t spmv_mul(int32_t a, int32_t b) { return (int32_t)((uin
 template <>
 __device__ inline int32_t spmv_add(int32_t a, int32_t b) { return (int32_t)((uint32_t)a + (uint32_t)b); }
 
-// Sequential sum of p[i0..i1) (index order), LDS reads eight, then four at a time.
-template <typename T>
+// Sequential sum of p[i0..i1) (index order), LDS reads U (a multiple of 8), then four at a time.
+template <int U, typename T>
 __device__ inline T lds_seq_sum(const T* __restrict__ p, int32_t i0, int32_t i1) {
   T sum = T(0);
   int32_t i = i0;
-  for (; i + 8 <= i1; i += 8) {
-    T a[8];
+  for (; i + U <= i1; i += U) {
+    T a[U];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) a[u] = p[i + u];
+    for (int u = 0; u < U; ++u) a[u] = p[i + u];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) sum = spmv_add(sum, a[u]);
+    for (int u = 0; u < U; ++u) sum = spmv_add(sum, a[u]);
   }
   for (; i + 4 <= i1; i += 4) {
     const T a0 = p[i], a1 = p[i + 1], a2 = p[i + 2], a3 = p[i + 3];
@@ -182,15 +182,16 @@ __global__ __launch_bounds__(kBlock) void spmv_windows_kernel(const int32_t* __r
       if (slot < (uint32_t)kMaxLongPerWindow) s_long[slot] = r;  // more only with malformed row pointers
       continue;
     }
-    // Eight LDS reads in flight: the longest row of a wave (tens of products, up to kLongRow) is a
+    // Sixteen LDS reads in flight: the longest row of a wave (tens of products, up to kLongRow) is a
     // chain of LDS latencies when each product is read and added by itself. With the bounds loaded
-    // early: 85K rows float 24.1 -> 11.0 us, 850K float 53.8 -> 41.2, 1M double 85 -> 73 (gathers
-    // from more than an XCD's L2), 3.2M double 313 -> 303. Windows of 2048 (fewer, longer row
-    // passes): 43.6, 78.5 and 318 us.
+    // early: 85K rows float 24.1 -> 10.5 us, 850K float 53.8 -> 40.6, 1M double 85 -> 73 (gathers
+    // from more than an XCD's L2), 3.2M double 313 -> 303. Eight: 10.9, 41.3, 73 and 304 us;
+    // eight with windows of 2048 (fewer, longer row passes): 43.6, 78.5 and 318 us for the last three.
+    // (The plan's row pass keeps eight: its rows hold at most kSeqRow.)
     // (the start is kept at or below the end, so that stepping by eight cannot wrap for row pointers
     // that are not monotone)
     const int32_t i1 = max(min(re - b, e - b), 0), i0 = min(max(rb - b, 0), i1);
-    const T sum = lds_seq_sum(s_prod, i0, i1);
+    const T sum = lds_seq_sum<16>(s_prod, i0, i1);
     __builtin_nontemporal_store(sum, y + r);
   }
   __syncthreads();
@@ -816,7 +817,7 @@ __global__ __launch_bounds__(SPAN / 8) void spmv_tile_rows(
     }
     const int32_t d = re - rb;
     float acc = 0.0f;
-    if (in && d <= kSeqRow) acc = lds_seq_sum(stage, rb - g.j0, min(re, g.j1) - g.j0);
+    if (in && d <= kSeqRow) acc = lds_seq_sum<8>(stage, rb - g.j0, min(re, g.j1) - g.j0);
     for (uint64_t m = __ballot(in && d > kSeqRow && re <= g.j1); m; m &= m - 1) {
       const int L = __builtin_ctzll(m);
       const int32_t lb = __builtin_amdgcn_readlane(rb, L) - g.j0, le = __builtin_amdgcn_readlane(re, L) - g.j0;
