@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kBlock) void spmv_windows_kernel(const int32_t* __r
     // from more than an XCD's L2), 3.2M double 313 -> 303. Eight: 10.9, 41.3, 73 and 304 us;
     // eight with windows of 2048 (fewer, longer row passes): 43.6, 78.5 and 318 us for the last three.
     // (The plan's row pass keeps eight: its rows hold at most kSeqRow.)
-    // (the start is kept at or below the end, so that stepping by eight cannot wrap for row pointers
+    // (the start is kept at or below the end, so that stepping by a batch cannot wrap for row pointers
     // that are not monotone)
     const int32_t i1 = max(min(re - b, e - b), 0), i0 = min(max(rb - b, 0), i1);
     const T sum = lds_seq_sum<16>(s_prod, i0, i1);
