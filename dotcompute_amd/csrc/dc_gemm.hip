@@ -5,11 +5,11 @@
 // bf16: v_mfma_f32_32x32x16_bf16 (bf16 inputs, fp32 accumulate).
 //
 // Kernels, by the shapes that take them:
-//   - gemm_f32_split_kernel<TM, TN, ...>: fp32, by six bf16 products per fp32 product; 256×256,
-//     128×128 or 64×64 macro tiles by the number of tiles.
-//   - gemm_f32_dma_kernel<64>: fp32 full 64-tiles, few of them with a short k, on the fp32
+//   - gemm_f32_split_kernel<TM, TN, ...>: fp32, by eight bf16 products per fp32 product; 256×128,
+//     128×128 or 64×64 macro tiles (the rule and its measurements: dc_gemm_route.hpp).
+//   - gemm_f32_dma_kernel<64>: fp32 full 64-tiles with a short k or few of them, on the fp32
 //     instructions: direct-to-LDS loads, double-buffered LDS, 4 waves of 32×32.
-//   - gemm_f32_kernel: the fp32 shapes left (fewer than 64 columns, one or two k tiles),
+//   - gemm_f32_kernel: the fp32 shapes left (fewer than 64 columns, at most 16 rows of B),
 //     bounds-checked 64×64 tiles on the fp32 instructions.
 //   - gemm_bf16_kernel<TM, TN, ...>: bf16, every shape. 256×256, 128×128 or 64×64 macro tiles by the
 //     number of tiles; direct-to-LDS loads of row-major A and B where rows are 16-byte aligned,
@@ -32,6 +32,7 @@
 #include <utility>
 
 #include "dc_device.hpp"
+#include "dc_gemm_route.hpp"
 #include "dc_internal.hpp"
 
 namespace {
@@ -62,8 +63,8 @@ __device__ inline TileCoord map_tile(int tiles_m, int tiles_n) {
 
 // ---------------------------------------------------------------------------------------------
 // fp32, full tiles (m, n multiples of T, k a multiple of 32): direct-to-LDS loads, no staging
-// registers and no transposing LDS stores. Launched with T = 64 for grids of at most one tile per CU
-// and k <= 1024 (1024^3: 19.7 us; see the dispatch).
+// registers and no transposing LDS stores. Launched with T = 64 for a short k or few tiles (1024^3:
+// 18.9 us; see dc_gemm_route.hpp).
 //   A tile [T rows][32 k] (128 B rows, unpadded): the 16-byte k-quad q of row R sits in slot
 //   q ^ ((R >> 1) & 7), so a fragment read (16 lanes = rows R0..R0+15 at one quad) touches 16
 //   distinct 16-byte bank groups.
@@ -721,16 +722,22 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
 
 // ---------------------------------------------------------------------------------------------
 // fp32 on the bf16 matrix cores: every fp32 value is the exact sum of three bf16 pieces,
-// x = x0 + x1 + x2 (x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1: 8 + 8 + 8 bits, rounded to
-// nearest, so |x1| <= 2^-9 |x| and |x2| <= 2^-18 |x|), and a·b is formed from the six products
-// a0 b0, a0 b1, a1 b0, a0 b2, a1 b1, a2 b0, each exact in fp32; the three left out are below
-// 2^-26 |a b|. 6 bf16 products cost 6/16 of one fp32 product on this chip's matrix cores, and a
-// 32×32×16 instruction adds 16 products per rounding where the fp32 one adds 2, so the result is
-// both faster and closer to the float64 product than the fp32 instructions' (relative error at
-// 8192^3 with normal inputs: 1.4e-6 against 1.6e-6). Measured: 8192^3 7.31 -> 4.50 ms (244
-// TFLOP/s where the fp32 instructions peak at 157), 4096^3 925 -> 561 us, 1537×2049×1023 144 -> 46 us.
-// Bound by the matrix cores at the clock that power allows (the 256-tile) and by what a workgroup's
-// barriers leave uncovered (the small tiles).
+// x = x0 + x1 + x2 (x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1, rounded to nearest, so |x1| <=
+// 2^-8 |x| and |x2| <= 2^-17 |x|), and a·b is formed from eight of the nine products of pieces, each
+// exact in fp32; the one left out, a2 b2, is at most 2^-34 |a b|. The sums of a0 b0 and those of the
+// seven small products stand in accumulators of their own and are added once, at the end: an
+// instruction's sum may be off by nearly an ulp (these matrix cores cut the addends at half an ulp of
+// the largest before they round), which matters 2^-7 times less in the small sums, and the large ones
+// are rounded once per 16 products where the fp32 instructions round each. So the result is closer to
+// the float64 product than theirs: relative error with normal inputs 8192^3 5.7e-7 against 1.62e-6,
+// 1537×2049×1023 1.3e-7 against 5.7e-7; a sum of one term is within 0.62 ulp (0.50). (All in one
+// accumulator, 256×256 tiles: 5.74 ms at 8192^3, 1.44e-6, one term up to an ulp off. Six products,
+// without a1 b2 and a2 b1: 4.6 ms, each product off by up to 2^-24 of it, one term up to 1.5 ulp.)
+// 8 bf16 products cost half of one fp32 product on this chip's matrix cores. Measured against the
+// kernels on the fp32 instructions: 8192^3 7.30 -> 6.02 ms (183 TFLOP/s where those instructions peak
+// at 157), 4096^3 925 -> 760 us, 1537×2049×1023 144 -> 53.5 us.
+// Bound by the matrix cores at the clock that power allows (large grids) and by what a workgroup's
+// barriers leave uncovered (small ones).
 //
 // Where the pieces do not hold the value: infinities and NaN (x - x0 is NaN, so the sum is), values
 // that round up to infinity in bf16 (likewise), and nonzero magnitudes below kSplitMin, whose lowest
@@ -746,7 +753,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
 // gemm_bf16_kernel). A tile's fp32 elements come through registers (16-byte loads at 4-byte alignment,
 // D tiles ahead: so no shape or alignment needs another kernel), are split and stored to LDS as three
 // bf16 planes, in the other of two buffers, while this tile's products run: about 7 VALU
-// instructions per element beside 48 (256-tile) or 24 MFMAs per wave and tile. LDS images per plane:
+// instructions per element beside 32 MFMAs (64-tiles: 8) per wave and tile. LDS images per plane:
 // - A: rows of 16 k (32 B); the 16-byte half h of row R sits at h ^ ((R >> 3) & 1), so a
 //   fragment read (16 rows at one half for each 16 lanes) touches 16 distinct 16-byte bank groups.
 // - B: k rows of TN n with the 64-byte blocks swizzled, read through ds_read_b64_tr_b16
@@ -887,7 +894,7 @@ struct SplitSmem {
 };
 
 template <int TM, int TN, int WM, int WN, int KS, int D>
-__global__ __launch_bounds__(64 * WM * WN * KS, (TM == 128 && KS == 1 ? 3 : 1)) void gemm_f32_split_kernel(
+__global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1)) void gemm_f32_split_kernel(
     const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N, int K, int tiles_m,
     int tiles_n) {
   constexpr int kWaves = WM * WN, kT = 64 * kWaves;
@@ -976,13 +983,13 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (TM == 128 && KS == 1 ? 3 : 1)) 
       boff[nt] = (uint32_t)offsetof(Smem, b) + (uint32_t)((8 * h + j) * 2 * TN) +
                  64u * (uint32_t)((kNT * wn + nt) ^ bswz(j)) + (uint32_t)(32 * cg + 8 * p4);
   }
-  f32x16 acc[kMT][kNT];
+  f32x16 acc[kMT][kNT], low[kMT][kNT];  // a0 b0's sums; the other products'
 #pragma unroll
   for (int i = 0; i < kMT; ++i)
 #pragma unroll
     for (int j = 0; j < kNT; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = low[i][j][v] = 0.0f;
   auto read_a = [&](int buf, int p, bf16x8 (&a)[kMT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int mt = 0; mt < kMT; ++mt)
@@ -998,29 +1005,32 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (TM == 128 && KS == 1 ? 3 : 1)) 
       b[nt] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
   };
-  auto mfmas = [&](const bf16x8 (&a)[kMT], const bf16x8 (&b)[kNT]) __attribute__((always_inline)) {
+  auto mfmas = [&](f32x16 (&sum)[kMT][kNT], const bf16x8 (&a)[kMT], const bf16x8 (&b)[kNT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < kNT; ++nt)
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
+        sum[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mt], b[nt], sum[mt][nt], 0, 0, 0);
   };
   // Fragments: plane 0 of B twice (the next tile's is read while this one's is still in use).
   bf16x8 a0[kMT], a1[kMT], a2[kMT], b0[2][kNT], b1[kNT], b2[kNT];
-  constexpr int kMfmas = 3 * kMT * kNT, kSplits = kA + kB;
-  // One k tile (buffer BUF) in two regions of three products each (small ones first), the barrier
-  // between them. First region: the reads of the planes that come last, and the split of the next tile
-  // (elements qa, qb) into the other buffer between the products. Second region: the reads of the
-  // next tile's first fragments between the products, so none of the LDS time is exposed.
+  constexpr int kMfmas = 5 * kMT * kNT, kSplits = kA + kB;  // of the first region
+  // One k tile (buffer BUF) in two regions, of five products (those with a2 or a1) and of three (a0's;
+  // a0 b0 is the last), the barrier between them. First region: the reads of the planes that come last,
+  // and the split of the next tile (elements qa, qb) into the other buffer between the products. Second
+  // region: the reads of the next tile's first fragments between the products, so none of the LDS time
+  // is exposed.
   auto first = [&](auto BUF, const dc::f32x4 (&qa)[kA], const dc::f32x4 (&qb)[kB]) __attribute__((always_inline)) {
     constexpr int kBuf = decltype(BUF)::value;
     __builtin_amdgcn_sched_barrier(0);
     read_a(kBuf, 0, a0);
     read_b(kBuf, 2, b2);
     split_tile(std::integral_constant<int, 1 - kBuf>{}, qa, qb);
-    mfmas(a2, b0[kBuf]);
-    mfmas(a1, b1);
-    mfmas(a1, b0[kBuf]);
+    mfmas(low, a2, b0[kBuf]);
+    mfmas(low, a2, b1);
+    mfmas(low, a1, b1);
+    mfmas(low, a1, b2);
+    mfmas(low, a1, b0[kBuf]);
     __builtin_amdgcn_sched_group_barrier(0x100, kMT + 2 * kNT, 0);
 #pragma unroll
     for (int i = 0; i < kMfmas; ++i) {
@@ -1036,9 +1046,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (TM == 128 && KS == 1 ? 3 : 1)) 
     read_a(kNext, 2, a2);
     read_b(kNext, 0, b0[kNext]);
     read_a(kNext, 1, a1);
-    mfmas(a0, b2);
-    mfmas(a0, b1);
-    mfmas(a0, b0[kBuf]);
+    mfmas(low, a0, b2);
+    mfmas(low, a0, b1);
+    mfmas(acc, a0, b0[kBuf]);
     read_b(kNext, 1, b1);
 #pragma unroll
     for (int i = 0; i < 2 * kMT * kNT; ++i) {
@@ -1052,8 +1062,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (TM == 128 && KS == 1 ? 3 : 1)) 
   constexpr std::integral_constant<int, 0> kBuf0{};
   constexpr std::integral_constant<int, 1> kBuf1{};
   static_assert(D == 1 || D == 2, "the loop is unrolled by two");
+  static_assert(TM <= 256, "the host checks 32-bit offsets in panels of 256 rows");
   // The group's last tile, the only one that can lie past K, comes first (checked loads); then tiles
-  // 0, 1, ...: step p > 0 is tile p - 1. The host sees to kt_count >= 2. Loads past the last step
+  // 0, 1, ...: step p > 0 is tile p - 1. The host sees to kt_count >= 2 (k > 16 KS). Loads past the last step
   // re-read its tile (unused): no branch in the loop, so its waits for memory cover just the tile
   // that is split next.
   load_checked(kt_count - 1, sa[0], sb[0]);
@@ -1088,15 +1099,20 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (TM == 128 && KS == 1 ? 3 : 1)) 
   };
   const bool early = __builtin_amdgcn_readfirstlane(s_redo) != 0;
   __builtin_assume(kt_count > 1);
-  int p = 0;
-  do {
-    if (early) break;
-    one(p, kBuf0);
-    if (p + 1 >= kt_count) break;
-    one(p + 1, kBuf1);
-    p += 2;
-  } while (p < kt_count);
+  if (!early) {
+    int p = 0;
+    do {  // (whole pairs: an exit between the two would cost copies of the accumulators)
+      one(p, kBuf0);
+      one(p + 1, kBuf1);
+      p += 2;
+    } while (p + 1 < kt_count);
+    if (p < kt_count) one(p, kBuf0);
+  }
   if (tiny < kTinyBits) s_tiny = 1;
+#pragma unroll
+  for (int i = 0; i < kMT * kNT; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[i / kNT][i % kNT][v] += low[i / kNT][i % kNT][v];
 
   if constexpr (KS > 1) {  // the groups' sums, added in group order by group 0
     constexpr int kSums = kT * kMT * kNT * 16;
@@ -1186,19 +1202,11 @@ void launch_bf16(dc_hip_ctx* ctx, const unsigned short* a, const unsigned short*
       a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
 }
 
-// The split kernel where its conditions hold (a whole tile of columns, two k tiles per group, and 32-bit
-// element offsets within a panel), else the checked fp32 kernel.
 template <int TM, int TN, int WM, int WN, int KS, int D>
-void launch_f32(dc_hip_ctx* ctx, const float* a, const float* b, float* c, int64_t m, int64_t n, int64_t k) {
-  if (n >= TN && k > 16 * KS && TM * k < INT32_MAX && 16 * n < INT32_MAX) {
-    const int tiles_m = (int)((m + TM - 1) / TM), tiles_n = (int)((n + TN - 1) / TN);
-    gemm_f32_split_kernel<TM, TN, WM, WN, KS, D><<<(unsigned)(tiles_m * tiles_n), 64 * WM * WN * KS, 0, ctx->stream>>>(
-        a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
-  } else {
-    const int tiles_m = (int)((m + 63) / 64), tiles_n = (int)((n + 63) / 64);
-    gemm_f32_kernel<kBKf32, true, 64><<<(unsigned)(tiles_m * tiles_n), kThreads, 0, ctx->stream>>>(
-        a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
-  }
+void launch_split(dc_hip_ctx* ctx, const float* a, const float* b, float* c, int64_t m, int64_t n, int64_t k) {
+  const int tiles_m = (int)((m + TM - 1) / TM), tiles_n = (int)((n + TN - 1) / TN);
+  gemm_f32_split_kernel<TM, TN, WM, WN, KS, D><<<(unsigned)(tiles_m * tiles_n), 64 * WM * WN * KS, 0, ctx->stream>>>(
+      a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
 }
 
 int32_t check_dims(int64_t m, int64_t n, int64_t k) {
@@ -1218,32 +1226,22 @@ DC_HIP_API int32_t dc_hip_gemm_f32(dc_hip_ctx* ctx, const float* a, const float*
   if (!c || (k > 0 && (!a || !b))) return DC_ERR_INVALID_ARGUMENT;
   DC_CTX_ENTER(ctx);
   if (k == 0) return dc::zero_async(ctx, c, (size_t)(m * n) * sizeof(float));
-  // The widest tile that still gives the chip enough workgroups, then a k dimension split over the
-  // wave groups of a workgroup. Measured (us; "xG": G groups; "f32": the fp32 instructions, direct-to-LDS):
-  //   8192^3: 256 4504, 128 5285, f32 7312;  4096^3: 561 / 658 / 925;  3500^3: 422 / 561, x2 572
-  //   3072x3072x1024 (144 tiles of 256, 576 of 128): 117 / 115, x2 134, f32 138
-  //   2048^3 (256 of 128): 218 / 104, x2 90.5, 64 118;  1536^3 (144 of 128): 167 / 76, x2 59, 64 64
-  //   1279x1281x641 (441 of 64): 128x2 29, 64 22.7, x2 20.8, x4 24.7
-  //   1023^3 (256 of 64): 25, x2 19.3, x4 19.5;  300x300x8000 (25 of 64): 164, x2 113, x4 99
-  //   full 64-tiles, f32 / best split: 256^3 6.2 / 8.8, 512^3 10.3 / 12, 1024^3 19.7 / 19.9,
-  //   512x512x4096 66 / 53: few tiles of a short k leave the split's longer start-up uncovered
-  const int64_t cus = std::max(1, ctx->cu_count);
-  auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
-  if (m % 64 == 0 && n % 64 == 0 && k % kBKd == 0 && dc::aligned16(a) && dc::aligned16(b) && tiles(64) <= cus && k <= 1024) {
-    // (each buffer range of the kernel, 64 rows of k floats or 32 rows of n, is below 2 GiB by then)
-    const int tiles_m = (int)(m / 64), tiles_n = (int)(n / 64);
-    gemm_f32_dma_kernel<64><<<(unsigned)(tiles_m * tiles_n), kThreads, 0, ctx->stream>>>(a, b, c, (int)m, (int)n, (int)k,
-                                                                                       tiles_m, tiles_n);
-  } else if (n >= 256 && 2 * tiles(256) > cus) {
-    launch_f32<256, 256, 2, 4, 1, 1>(ctx, a, b, c, m, n, k);
-  } else if (n >= 128 && tiles(128) > cus) {
-    launch_f32<128, 128, 2, 2, 1, 1>(ctx, a, b, c, m, n, k);
-  } else if (n >= 128 && 2 * tiles(128) > cus && k >= 256) {
-    launch_f32<128, 128, 2, 2, 2, 2>(ctx, a, b, c, m, n, k);
-  } else if (tiles(64) > cus || k < 1536) {
-    launch_f32<64, 64, 2, 2, 2, 2>(ctx, a, b, c, m, n, k);
-  } else {
-    launch_f32<64, 64, 2, 2, 4, 2>(ctx, a, b, c, m, n, k);
+  const int tiles_m = (int)((m + 63) / 64), tiles_n = (int)((n + 63) / 64);
+  switch (dc::f32_gemm_kernel(m, n, k, dc::aligned16(a) && dc::aligned16(b), std::max(1, ctx->cu_count))) {
+    case dc::F32Gemm::kDma64:
+      gemm_f32_dma_kernel<64><<<(unsigned)(tiles_m * tiles_n), kThreads, 0, ctx->stream>>>(a, b, c, (int)m, (int)n, (int)k,
+                                                                                         tiles_m, tiles_n);
+      break;
+    case dc::F32Gemm::kChecked64:
+      gemm_f32_kernel<kBKf32, true, 64><<<(unsigned)(tiles_m * tiles_n), kThreads, 0, ctx->stream>>>(
+          a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
+      break;
+    case dc::F32Gemm::kSplit256x128: launch_split<256, 128, 4, 2, 1, 1>(ctx, a, b, c, m, n, k); break;
+    case dc::F32Gemm::kSplit128: launch_split<128, 128, 2, 2, 1, 1>(ctx, a, b, c, m, n, k); break;
+    case dc::F32Gemm::kSplit128x2: launch_split<128, 128, 2, 2, 2, 2>(ctx, a, b, c, m, n, k); break;
+    case dc::F32Gemm::kSplit64: launch_split<64, 64, 2, 2, 1, 2>(ctx, a, b, c, m, n, k); break;
+    case dc::F32Gemm::kSplit64x2: launch_split<64, 64, 2, 2, 2, 2>(ctx, a, b, c, m, n, k); break;
+    case dc::F32Gemm::kSplit64x4: launch_split<64, 64, 2, 2, 4, 2>(ctx, a, b, c, m, n, k); break;
   }
   return dc::last_launch_status();
 }

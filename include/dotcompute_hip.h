@@ -455,8 +455,9 @@ DC_HIP_API int32_t dc_hip_linq_where_select_minmax_i32(dc_hip_ctx* ctx, const dc
  * OptimizedMatrixMultiplyKernel.cs:72-96), MatrixOperations.MultiplyAsync / MultiplyOnGPUAsync
  * (src/Extensions/DotCompute.Algorithms/LinearAlgebra/Operations/MatrixOperations.cs:28-64,359-440)
  * and the 16×16 tiled string kernels (LinearAlgebra/MatrixKernels.cs:11-80).
- * f32: fp32 inputs, fp32 accumulate; each product from three exact bf16 pieces per operand (error
- *      below 2^-26 of it) or by the fp32 matrix instructions, by shape and value range.
+ * f32: fp32 inputs, fp32 accumulate; each product from three exact bf16 pieces per operand (within
+ *      2^-34 of it; a sum of one term within 0.62 ulp) or by the fp32 matrix instructions, by shape and
+ *      value range.
  * bf16: bf16 inputs (uint16 bit patterns), bf16 MFMA, fp32 accumulate and output.
  * Leading dimensions equal the row lengths (k for A, n for B and C).
  * ------------------------------------------------------------------------------------------- */

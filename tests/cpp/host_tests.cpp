@@ -9,6 +9,7 @@
 #include <cstring>
 #include <random>
 
+#include "../../dotcompute_amd/csrc/dc_gemm_route.hpp"
 #include "DotCompute/Algorithms.hpp"
 #include "DotCompute/Linq.hpp"
 #include "DotCompute/Runtime.hpp"
@@ -209,6 +210,28 @@ std::shared_ptr<Backends::Hip::HipAccelerator> Gpu() {
 }  // namespace
 
 // ============================== CPU: fusion planner ==============================================
+
+// The shapes of tests/test_gpu_gemm.py that are there for one kernel each, and each rule's edges.
+TEST_CPU(GemmF32_EachShapeTakesItsKernel) {
+  using dc::F32Gemm;
+  struct Row {
+    int64_t m, n, k;
+    F32Gemm want;
+  };
+  const Row rows[] = {
+      {2570, 2571, 515, F32Gemm::kSplit256x128}, {2824, 3083, 67, F32Gemm::kSplit128}, {1799, 1911, 771, F32Gemm::kSplit128x2},
+      {300, 333, 61, F32Gemm::kSplit64}, {300, 333, 257, F32Gemm::kSplit64x2}, {129, 131, 1537, F32Gemm::kSplit64x4},
+      {128, 192, 64, F32Gemm::kDma64}, {65, 60, 40, F32Gemm::kChecked64}, {65, 64, 17, F32Gemm::kSplit64},
+      {65, 64, 16, F32Gemm::kChecked64}, {64, 100000, 256, F32Gemm::kSplit64}, {2048, 2048, 64, F32Gemm::kDma64},
+      {4096, 4096, 128, F32Gemm::kSplit128}, {64, 64, 4096, F32Gemm::kSplit64x4}, {8192, 8192, 8192, F32Gemm::kSplit256x128},
+      // past the 32-bit offsets of the split kernels and the buffer ranges of the direct ones
+      {128, 128, INT32_MAX / 256 + 1, F32Gemm::kChecked64}, {64, 1 << 24, 64, F32Gemm::kSplit64},
+      {1, INT32_MAX / 16 + 1, 64, F32Gemm::kChecked64}};
+  for (const Row& r : rows)
+    if (dc::f32_gemm_kernel(r.m, r.n, r.k, true, 256) != r.want)
+      throw dctest::Failure(std::to_string(r.m) + "x" + std::to_string(r.n) + "x" + std::to_string(r.k));
+  CHECK(dc::f32_gemm_kernel(128, 192, 64, false, 256) == F32Gemm::kSplit64);
+}
 
 TEST_CPU(planner_emits_the_benchmark_chain) {
   auto x = Param();

@@ -194,11 +194,15 @@ def test_gemm_bf16_ragged_tiles(ctx, shape):
     assert np.array_equal(c0, c[0])
 
 
-# One shape per tile choice of the fp32 dispatch (on 256 CUs), rows, columns and last k tile ragged:
-# 256-tiles, 128-tiles with one and two k groups, 64-tiles with two and four; the smallest k that
-# the two- and four-group kernels take, and one less.
-@pytest.mark.parametrize("shape", [(2824, 3083, 50), (2200, 2057, 131), (1799, 1911, 257), (300, 333, 61),
-                                   (129, 131, 1537), (65, 64, 33), (65, 64, 32), (200, 1000, 49)])
+# One shape per kernel of the fp32 dispatch (on 256 CUs): split 256x128, 128, 128 with two k groups, 64,
+# 64 with two and four, each with ragged rows, columns and last k tile; the fp32 instructions on full and
+# on ragged tiles. (host_tests.cpp checks that each shape takes the kernel it is here for.)
+F32_KERNELS = [(2570, 2571, 515), (2824, 3083, 67), (1799, 1911, 771), (300, 333, 61), (300, 333, 257),
+               (129, 131, 1537), (128, 192, 64), (65, 60, 40)]
+
+
+# (and the smallest k that the split kernels take, one less, and two shapes of few columns or rows)
+@pytest.mark.parametrize("shape", F32_KERNELS + [(65, 64, 17), (65, 64, 16), (200, 64, 49), (64, 1000, 49)])
 def test_gemm_f32_split_tiles(ctx, shape):
     m, n, k = shape
     a, b = make_inputs(m, n, k)
@@ -239,3 +243,58 @@ def test_gemm_f32_split_permutation_exact(ctx):
     perm = np.eye(n, dtype=np.float32)[np.random.default_rng(1).permutation(n)]
     assert np.array_equal(run_gemm(ctx, perm, a), perm @ a)
     assert np.array_equal(run_gemm(ctx, a, perm), a @ perm)
+
+
+@pytest.mark.parametrize("shape", F32_KERNELS)
+def test_gemm_f32_single_terms(ctx, shape):
+    """Scaled rows and columns: one product per entry, which the sum must hold as its roundings allow.
+
+    The sum of the large products is one product and exact. The seven small products are below 2^-6.9
+    |ab| in all; each addition of theirs is off by an ulp (2^-23 of the sum) at most, so with the product
+    left out (2^-34) they are off by less than 2^-27 |ab|, an eighth of an ulp; the two sums are added with
+    one rounding, half an ulp."""
+    m, n, k = shape
+    rng = np.random.default_rng(m)
+
+    def values(*size):  # every mantissa bit, four binades, and 1.0038986 (pieces 1, 2^-8 and -2^-17) among them
+        x = rng.uniform(1.0, 2.0, size) * 2.0 ** rng.integers(-2, 2, size) * rng.choice([-1.0, 1.0], size)
+        x[rng.uniform(size=size) < 0.1] = 1.0038986
+        return x.astype(np.float32)
+
+    def check(got, exact):
+        ulp = np.spacing(np.abs(exact).astype(np.float32)).astype(np.float64)
+        assert np.max(np.abs(got - exact) / ulp) <= 0.5 + 2.0 ** -3
+
+    place, factor = rng.integers(0, k, m), values(m)
+    a, b = np.zeros((m, k), np.float32), values(k, n)
+    a[np.arange(m), place] = factor
+    check(run_gemm(ctx, a, b), factor[:, None].astype(np.float64) * b[place])
+    place, factor = rng.integers(0, k, n), values(n)
+    a, b = values(m, k), np.zeros((k, n), np.float32)
+    b[place, np.arange(n)] = factor
+    check(run_gemm(ctx, a, b), factor.astype(np.float64) * a[:, place])
+
+
+@pytest.mark.parametrize("shape", F32_KERNELS)
+def test_gemm_f32_integers_exact(ctx, shape):
+    """9-bit integers, 60 at most per row: every partial sum is below 2^24, so any order is exact, and
+    every value but the multiples of two has a second piece."""
+    m, n, k = shape
+    rng = np.random.default_rng(n)
+    a = rng.integers(-511, 512, (m, k)) * (rng.uniform(size=(m, k)) < 50 / max(k, 50))
+    for row in a:
+        row[np.flatnonzero(row)[60:]] = 0
+    b = rng.integers(-511, 512, (k, n))
+    assert np.array_equal(run_gemm(ctx, a.astype(np.float32), b.astype(np.float32)), (a @ b).astype(np.float32))
+
+
+@pytest.mark.parametrize("shape", F32_KERNELS + [(1537, 2049, 1023)])
+def test_gemm_f32_error_of_a_float32_sum(ctx, shape):
+    """Normal inputs: k roundings of partial sums, each of rms 2^-24 / sqrt(3) of a sum whose mean square
+    is half of the last one's, make 2^-24 sqrt(k / 6) in the 2-norm; every second-order product of
+    pieces (rms 2^-19 of a product) would show."""
+    m, n, k = shape
+    rng = np.random.default_rng(k)
+    a, b = rng.standard_normal((m, k), np.float32), rng.standard_normal((k, n), np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.linalg.norm(run_gemm(ctx, a, b) - ref) <= 2.0 ** -24 * (k / 6) ** 0.5 * np.linalg.norm(ref)
