@@ -741,13 +741,18 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
 //
 // Where the pieces do not hold the value: infinities and NaN (x - x0 is NaN, so the sum is), values
 // that round up to infinity in bf16 (likewise), and nonzero magnitudes below kSplitMin, whose lowest
-// pieces fall below bf16's subnormals (an error below 2^-134 each). A tile whose sums are not all
-// finite, or that met such small values and has a sum they could have moved by more than 2^-26 of
-// itself, computes itself again with v_mfma_f32_32x32x2_f32 (f32_tile_direct below), so those inputs
-// give what the fp32 instructions give. (8192^3 with every value of A near 2^-110: 10.7 ms against
-// 7.3 ms on the fp32 instructions alone; with a tenth of them scattered: 5.3 ms.) bf16 subnormals and
-// products down to the fp32 subnormals are kept by the matrix cores (measured), so results near
-// 2^-126 are as exact as before.
+// pieces fall below bf16's subnormals (an error below 2^-134 each). A sum that is not finite, or that
+// such small values in its row of A or column of B could have moved by more than 2^-32 of itself, is
+// formed again with v_mfma_f32_32x32x2_f32 (f32_blocks_direct below), and only it is stored again: those
+// inputs give what the fp32 instructions give, and every other sum has the same bits whatever the rest
+// of its tile holds. Tiles in which nothing would stand are not formed by pieces at all: every row of
+// A past kSplitMax in the first k tile, or that tile of A or of B nonzero and below kSplitMin throughout
+// (the one case in which a sum's arithmetic depends on its tile). Measured at 8192^3 (fp32 instructions
+// alone 7.3 ms; 6.1 without such values): an infinity in one row of every 256 8.3 ms, in every 16th row
+// 19.4 (every block of 32×32 is formed twice); half of A at -3.4e38, or all of it NaN or near 2^-110, 13.2;
+// a tenth of A's elements near 2^-110 6.2, with half the columns of B zero 6.6. At 1537×2049×1023 (144 us;
+// 55.6): 123, 132, 82, 58 and 80 us. bf16 subnormals and products down to the fp32 subnormals are kept by
+// the matrix cores (measured), so results near 2^-126 are as exact as before.
 //
 // Macro tile TM×TN, KS groups of WM×WN waves that take the k tiles (16 k each) in turn (as
 // gemm_bf16_kernel). A tile's fp32 elements come through registers (16-byte loads at 4-byte alignment,
@@ -760,6 +765,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
 //   (as gemm_bf16_kernel).
 // ---------------------------------------------------------------------------------------------
 constexpr float kSplitMin = 0x1p-102f;
+constexpr float kSplitMax = 0x1.fefffep127f;  // the largest magnitude that does not round to infinity in bf16
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -771,15 +777,15 @@ __device__ __attribute__((always_inline)) inline void for_each_index(F&& f, std:
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-// The three bf16 pieces of four values, packed; *tiny becomes the smallest (2|x| as bits) - 1 seen
-// (all ones for x = 0).
-__device__ inline void split_quad(dc::f32x4 x, u32x2 (&piece)[3], uint32_t* tiny) {
+// The three bf16 pieces of four values, packed; *big becomes the largest 2|x| (as bits) seen, *tiny the
+// smallest less 1 (all ones for x = 0).
+__device__ inline void split_quad(dc::f32x4 x, u32x2 (&piece)[3], uint32_t* big, uint32_t* tiny) {
   f32x2 v[2] = {{x.x, x.y}, {x.z, x.w}};
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const uint32_t t0 = (__builtin_bit_cast(uint32_t, v[i].x) << 1) - 1u;
-    const uint32_t t1 = (__builtin_bit_cast(uint32_t, v[i].y) << 1) - 1u;
-    *tiny = min(*tiny, min(t0, t1));
+    const uint32_t u0 = __builtin_bit_cast(uint32_t, v[i].x) << 1, u1 = __builtin_bit_cast(uint32_t, v[i].y) << 1;
+    *big = max(*big, max(u0, u1));
+    *tiny = min(*tiny, min(u0 - 1u, u1 - 1u));
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v[i], bf16x2));
@@ -792,99 +798,120 @@ __device__ inline void split_quad(dc::f32x4 x, u32x2 (&piece)[3], uint32_t* tiny
   }
 }
 
-// One workgroup's C tile with the fp32 matrix instructions, into acc (waves of group 0; every wave of the
-// workgroup takes part in the barriers). Operands are staged k-row by k-row in LDS (`la`: 16 rows
-// of TM + 32, `lb`: 16 rows of TN + 32 floats); every load is checked.
-template <int TM, int TN, int kMT, int kNT, int kThreadsPerGroup>
-__device__ __attribute__((always_inline)) inline void f32_tile_direct(const float* __restrict__ A, const float* __restrict__ B, int M,
-                                                          int N, int K, int m0, int n0, int t, bool active, int wm,
-                                                          int wn, float* la, float* lb, f32x16 (&acc)[kMT][kNT]) {
-  constexpr int kA = TM * 16 / kThreadsPerGroup, kB = TN * 16 / kThreadsPerGroup;
-  constexpr int kPitchA = TM + 32, kPitchB = TN + 32;
-  const int lane = t & 63, r = lane & 31, h = lane >> 5;
-  float ea[kA], eb[kB];
-  auto load = [&](int k0) __attribute__((always_inline)) {
+// A wave's 32×32 blocks (bits mt·kNT + nt of `need`, uniform) at row0, col0 of C with the fp32 matrix
+// instructions, into acc. Fragments come straight from global memory, two steps of 32 k's in flight, so
+// waves with nothing to do cost the others nothing: no LDS, no barrier. Lane group h takes the k's [16h,
+// 16h + 16) of a step, so a step's loads of A use whole 128-byte lines at once. Rows past M re-read the
+// last one; every column exists.
+template <int kMT, int kNT>
+__device__ __attribute__((always_inline)) inline void f32_blocks_direct(const float* __restrict__ A,
+                                                                        const float* __restrict__ B, int M, int N, int K,
+                                                                        int row0, int col0, int lane, uint32_t need,
+                                                                        f32x16 (&acc)[kMT][kNT]) {
+  constexpr int kDepth = 2, kStep = 32, kHalf = kStep / 2;
+  const int r = lane & 31, h = lane >> 5;
+  const float* pa[kMT];
 #pragma unroll
-    for (int i = 0; i < kA; ++i) {
-      const int e = i * kThreadsPerGroup + t, m = m0 + e / 16, k = k0 + e % 16;
-      ea[i] = active && m < M && k < K ? A[(size_t)m * K + k] : 0.0f;
-    }
+  for (int mt = 0; mt < kMT; ++mt) pa[mt] = A + (size_t)min(row0 + mt * 32 + r, M - 1) * K + kHalf * h;
+  const float* pb = B + (size_t)(kHalf * h) * N + col0 + r;
+  dc::f32x4 a[kDepth][kMT][kHalf / 4];
+  float b[kDepth][kNT][kHalf];
+  auto load = [&](int s, dc::f32x4 (&fa)[kMT][kHalf / 4], float (&fb)[kNT][kHalf]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kB; ++i) {
-      const int e = i * kThreadsPerGroup + t, k = k0 + e / TN, n = n0 + e % TN;
-      eb[i] = active && k < K && n < N ? B[(size_t)k * N + n] : 0.0f;
-    }
+    for (int i = 0; i < kMT * kHalf / 4; ++i)
+      fa[i / (kHalf / 4)][i % (kHalf / 4)] =
+          *reinterpret_cast<const f32x4_any*>(pa[i / (kHalf / 4)] + kStep * s + 4 * (i % (kHalf / 4)));
+#pragma unroll
+    for (int i = 0; i < kHalf * kNT; ++i) fb[i % kNT][i / kNT] = pb[(size_t)(kStep * s + i / kNT) * N + 32 * (i % kNT)];
+  };
+  auto multiply = [&](const dc::f32x4 (&fa)[kMT][kHalf / 4], const float (&fb)[kNT][kHalf]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kMT * kNT; ++i)
+      if (need >> i & 1u)
+#pragma unroll
+        for (int kk = 0; kk < kHalf; ++kk)
+          acc[i / kNT][i % kNT] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i / kNT][kk >> 2][kk & 3], fb[i % kNT][kk],
+                                                                       acc[i / kNT][i % kNT], 0, 0, 0);
   };
 #pragma unroll
-  for (int i = 0; i < kMT * kNT; ++i)
+  for (int i = 0; i < kMT * kNT * 16; ++i) acc[i / 16 / kNT][i / 16 % kNT][i % 16] = 0.0f;
+  const int whole = K / kStep;  // steps
+  int s = 0;
+  if (whole >= kDepth) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[i / kNT][i % kNT][v] = 0.0f;
-  load(0);
+    for (int d = 0; d < kDepth; ++d) load(d, a[d], b[d]);
 #pragma unroll 1
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    __syncthreads();
-    if (active) {
+    for (; s + kDepth <= whole; s += kDepth)
 #pragma unroll
-      for (int i = 0; i < kA; ++i) {
-        const int e = i * kThreadsPerGroup + t;
-        la[(e % 16) * kPitchA + e / 16] = ea[i];
+      for (int d = 0; d < kDepth; ++d) {
+        multiply(a[d], b[d]);
+        load(min(s + kDepth + d, whole - 1), a[d], b[d]);
       }
+  }
+#pragma unroll 1
+  for (; s < whole; ++s) {
+    load(s, a[0], b[0]);
+    multiply(a[0], b[0]);
+  }
+  if (K % kStep != 0) {
+    const int left = K - kStep * whole - kHalf * h;  // of the lane group's k's
 #pragma unroll
-      for (int i = 0; i < kB; ++i) {
-        const int e = i * kThreadsPerGroup + t;
-        lb[(e / TN) * kPitchB + e % TN] = eb[i];
-      }
-    }
-    __syncthreads();
-    if (k0 + 16 < K) load(k0 + 16);
-    if (active) {
+    for (int i = 0; i < kMT * kHalf; ++i)
+      a[0][i / kHalf][i / 4 % (kHalf / 4)][i % 4] = i % kHalf < left ? pa[i / kHalf][kStep * whole + i % kHalf] : 0.0f;
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-        float a[kMT], b[kNT];
-#pragma unroll
-        for (int mt = 0; mt < kMT; ++mt) a[mt] = la[(2 * kk + h) * kPitchA + (wm * kMT + mt) * 32 + r];
-#pragma unroll
-        for (int nt = 0; nt < kNT; ++nt) b[nt] = lb[(2 * kk + h) * kPitchB + (wn * kNT + nt) * 32 + r];
-#pragma unroll
-        for (int mt = 0; mt < kMT; ++mt)
-#pragma unroll
-          for (int nt = 0; nt < kNT; ++nt)
-            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
-      }
-    }
+    for (int i = 0; i < kNT * kHalf; ++i)
+      b[0][i / kHalf][i % kHalf] = i % kHalf < left ? pb[(size_t)(kStep * whole + i % kHalf) * N + 32 * (i / kHalf)] : 0.0f;
+    multiply(a[0], b[0]);
   }
 }
 
-// A thread's share of the largest magnitude among A[0, count) and the K rows of TN columns at B.
+// Whether a magnitude (as 2|x|'s bits - 1; zero: all ones) is nonzero and below kSplitMin.
+constexpr uint32_t kTinyBits = 2u * __builtin_bit_cast(uint32_t, kSplitMin) - 1u;
+
+// For each of `rows` rows of K at A and each of TN columns of the K rows at B: the bits of its largest
+// magnitude into stat[row], stat[TM + column], and 1 into stat[TM + TN + ...] if it holds a nonzero
+// one below kSplitMin. By the whole workgroup; stat is zero before.
 template <int TM, int TN, int kThreadsPerBlock>
-__device__ inline float panel_max(const float* __restrict__ A, size_t count, const float* __restrict__ B, int N, int K,
-                                  int tid) {
-  constexpr int kIn = 8;  // 16-byte loads in flight; the last ones re-read the end
-  float big = 0.0f;
+__device__ inline void panel_stats(const float* __restrict__ A, int rows, const float* __restrict__ B, int N, int K, int tid,
+                                   uint32_t* stat) {
+  constexpr int kIn = 8;  // 16-byte loads in flight; the last ones re-read the end (K >= 4)
   auto take = [&](const float* p) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4_any*>(p); };
-  auto fold = [&](dc::f32x4 x) __attribute__((always_inline)) {
-    const float lo = __builtin_fmaxf(__builtin_fabsf(x.x), __builtin_fabsf(x.y));
-    big = __builtin_fmaxf(big, __builtin_fmaxf(lo, __builtin_fmaxf(__builtin_fabsf(x.z), __builtin_fabsf(x.w))));
+  auto fold = [&](float x, uint32_t& big, uint32_t& tiny) __attribute__((always_inline)) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x) << 1;
+    big = max(big, u);
+    tiny = min(tiny, u - 1u);
+  };
+  auto put = [&](int i, uint32_t big, uint32_t tiny) __attribute__((always_inline)) {
+    atomicMax(&stat[i], big >> 1);
+    if (tiny < kTinyBits) stat[TM + TN + i] = 1u;
   };
 #pragma unroll 1
-  for (size_t i = 4 * tid; i < count; i += 4 * kIn * kThreadsPerBlock) {
-    dc::f32x4 x[kIn];
+  for (int row = tid >> 6; row < rows; row += kThreadsPerBlock / 64) {  // a wave per row
+    const float* p = A + (size_t)row * K;
+    uint32_t big = 0, tiny = 0xFFFFFFFFu;
+#pragma unroll 1
+    for (int k = 4 * (tid & 63); k < K; k += 256 * kIn) {
+      dc::f32x4 x[kIn];
 #pragma unroll
-    for (int u = 0; u < kIn; ++u) x[u] = take(A + min(i + 4 * u * kThreadsPerBlock, count - 4));
+      for (int u = 0; u < kIn; ++u) x[u] = take(p + min(k + 256 * u, K - 4));
 #pragma unroll
-    for (int u = 0; u < kIn; ++u) fold(x[u]);
+      for (int u = 0; u < 4 * kIn; ++u) fold(x[u / 4][u % 4], big, tiny);
+    }
+    put(row, big, tiny);
   }
   constexpr int kRows = 4 * kThreadsPerBlock / TN;
-  B += 4 * (tid % (TN / 4));
+  const int col = 4 * (tid % (TN / 4));
+  uint32_t big[4] = {}, tiny[4] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
 #pragma unroll 1
   for (int k = tid / (TN / 4); k < K; k += kIn * kRows) {
     dc::f32x4 x[kIn];
 #pragma unroll
-    for (int u = 0; u < kIn; ++u) x[u] = take(B + (size_t)min(k + u * kRows, K - 1) * N);
+    for (int u = 0; u < kIn; ++u) x[u] = take(B + col + (size_t)min(k + u * kRows, K - 1) * N);
 #pragma unroll
-    for (int u = 0; u < kIn; ++u) fold(x[u]);
+    for (int u = 0; u < 4 * kIn; ++u) fold(x[u / 4][u % 4], big[u % 4], tiny[u % 4]);
   }
-  return big;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) put(TM + col + e, big[e], tiny[e]);
 }
 
 template <int TM, int TN>
@@ -903,8 +930,8 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
   constexpr int kA = TM * 4 / kT, kB = TN * 4 / kT;  // quads per thread and k tile
   using Smem = SplitSmem<TM, TN>;
   __shared__ __align__(16) Smem sms[KS];
-  __shared__ int s_redo, s_tiny;
-  __shared__ uint32_t s_big;
+  __shared__ int s_redo, s_tiny, s_low;
+  __shared__ uint32_t s_seen, s_big;
   const TileCoord tc = map_tile(tiles_m, tiles_n);
   const int m0 = tc.tm * TM;
   const int n0 = min(tc.tn * TN, N - TN);  // the last tile ends at N (N >= TN, by the host)
@@ -931,7 +958,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
     wb[i] = (uint32_t)(krow * TN + 32 * ((nq >> 3) ^ bswz(krow)) + 4 * (nq & 7));
   }
   dc::f32x4 sa[D][kA], sb[D][kB];  // D tiles of elements in flight
-  uint32_t tiny = 0xFFFFFFFFu;     // over the lane's elements: see split_quad
+  uint32_t big = 0, tiny = 0xFFFFFFFFu;  // over the lane's elements: see split_quad
   // The group's k tile KT, every element of which exists.
   auto load_tile = [&](int KT, dc::f32x4 (&qa)[kA], dc::f32x4 (&qb)[kB]) __attribute__((always_inline)) {
     const int k0 = (KT * KS + group) * kBK;
@@ -960,13 +987,13 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
     u32x2 piece[3];
 #pragma unroll
     for (int i = 0; i < kA; ++i) {
-      split_quad(qa[i], piece, &tiny);
+      split_quad(qa[i], piece, &big, &tiny);
 #pragma unroll
       for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(&sm.a[kBuf][p][0] + wa[i]) = piece[p];
     }
 #pragma unroll
     for (int i = 0; i < kB; ++i) {
-      split_quad(qb[i], piece, &tiny);
+      split_quad(qb[i], piece, &big, &tiny);
 #pragma unroll
       for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(&sm.b[kBuf][p][0][0] + wb[i]) = piece[p];
     }
@@ -1035,7 +1062,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
 #pragma unroll
     for (int i = 0; i < kMfmas; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, (26 * kSplits + kMfmas - 1) / kMfmas, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, (28 * kSplits + kMfmas - 1) / kMfmas, 0);
       __builtin_amdgcn_sched_group_barrier(0x200, (3 * kSplits + kMfmas - 1) / kMfmas, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1057,8 +1084,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  if (tid == 0) s_redo = s_tiny = s_big = 0;
-  constexpr uint32_t kTinyBits = 2u * __builtin_bit_cast(uint32_t, kSplitMin) - 1u;
+  if (tid == 0) s_redo = s_tiny = s_low = s_seen = s_big = 0;
   constexpr std::integral_constant<int, 0> kBuf0{};
   constexpr std::integral_constant<int, 1> kBuf1{};
   static_assert(D == 1 || D == 2, "the loop is unrolled by two");
@@ -1069,16 +1095,29 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
   // that is split next.
   load_checked(kt_count - 1, sa[0], sb[0]);
   split_tile(kBuf0, sa[0], sb[0]);
-  __syncthreads();  // s_redo, s_tiny, s_big are set
-  {  // nothing but small values in a wave's share of the first tile: they are no exception here
+  __syncthreads();  // the flags are set
+  {  // bits: A's first tiles hold a nonzero value, one of at least kSplitMin; B's; a row of A's without a
+     // value past kSplitMax
     float big_a = 0.0f, big_b = 0.0f;
+    bool clean = false;
 #pragma unroll
-    for (int i = 0; i < 4 * kA; ++i) big_a = __builtin_fmaxf(big_a, __builtin_fabsf(sa[0][i / 4][i % 4]));
+    for (int i = 0; i < kA; ++i) {
+      bool past = false;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        big_a = __builtin_fmaxf(big_a, __builtin_fabsf(sa[0][i][e]));
+        past |= !(__builtin_fabsf(sa[0][i][e]) <= kSplitMax);
+      }
+      uint64_t m = __ballot(past);  // four lanes hold a row
+      m |= m >> 1;
+      m |= m >> 2;
+      clean |= (~m & 0x1111111111111111ull) != 0;
+    }
 #pragma unroll
     for (int i = 0; i < 4 * kB; ++i) big_b = __builtin_fmaxf(big_b, __builtin_fabsf(sb[0][i / 4][i % 4]));
-    const bool small_a = __any(big_a > 0.0f) && !__any(big_a >= kSplitMin);
-    const bool small_b = __any(big_b > 0.0f) && !__any(big_b >= kSplitMin);
-    if (small_a || small_b) s_redo = 1;
+    const uint32_t seen = (__any(big_a > 0.0f) ? 1u : 0u) | (__any(big_a >= kSplitMin) ? 2u : 0u) |
+                          (__any(big_b > 0.0f) ? 4u : 0u) | (__any(big_b >= kSplitMin) ? 8u : 0u) | (clean ? 16u : 0u);
+    if (lane == 0) atomicOr(&s_seen, seen);
   }
   for_each_index([&](auto I) __attribute__((always_inline)) {
     load_tile(min(I.value, kt_count - 2), sa[(1 + I.value) % D], sb[(1 + I.value) % D]);
@@ -1097,7 +1136,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
     load_tile(min(p + D, kt_count - 2), sa[set], sb[set]);
     second(I);
   };
-  const bool early = __builtin_amdgcn_readfirstlane(s_redo) != 0;
+  // Nothing but small values in all of the first tiles (they are no exception here), or no sum that stands.
+  const uint32_t seen = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_seen);
+  const bool early = (seen & 3u) == 1u || (seen & 12u) == 4u || (seen & 16u) == 0u;
   __builtin_assume(kt_count > 1);
   if (!early) {
     int p = 0;
@@ -1132,46 +1173,88 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
       }
   }
   __syncthreads();
-  float least = 0.0f;  // sums below this may have lost more than 2^-26 of themselves to small values
-  if (s_tiny && !early) {  // uniform
-    const float big = panel_max<TM, TN, kT * KS>(A + (size_t)m0 * K, (size_t)min(TM, M - m0) * K, B + n0, N, K, tid);
-    atomicMax(&s_big, __builtin_bit_cast(uint32_t, big));
+  // Which sums stand: finite, and not moved by the pieces that small values lost, 2^-134 at most each, by
+  // more than 2^-32 of themselves. By row and column, so that a sum's arithmetic depends on no other's.
+  uint32_t* stat = reinterpret_cast<uint32_t*>(&sms[0]);
+  static_assert(sizeof(Smem) >= 2 * (TM + TN) * sizeof(uint32_t), "the rows' and columns' figures fit in the buffers");
+  constexpr float kLost = 0x1p-102f;
+  bool scan = s_tiny != 0 && !early;  // uniform, as all of this
+  if (scan) {  // unless every sum stands whatever its row and column hold
+    atomicMax(&s_big, big >> 1);
     __syncthreads();
-    least = __builtin_bit_cast(float, s_big) * (float)K * 0x1p-107f;  // 2 K lost pieces of at most 2^-134
+    const float least = __builtin_bit_cast(float, s_big) * 2.0f * ((float)K * kLost);
+    bool low = false;
+#pragma unroll
+    for (int i = 0; i < kMT * kNT * 16; ++i)
+      low |= !(__builtin_fabsf(acc[i / 16 / kNT][i / 16 % kNT][i % 16]) >= least);  // (NaN: not known to)
+    if (group == 0 && low) s_low = 1;
+    __syncthreads();
+    scan = s_low != 0;
   }
+  if (scan) {
+    for (int i = tid; i < 2 * (TM + TN); i += kT * KS) stat[i] = 0;
+    __syncthreads();
+    panel_stats<TM, TN, kT * KS>(A + (size_t)m0 * K, min(TM, M - m0), B + n0, N, K, tid, stat);
+    __syncthreads();
+  }
+  auto stands = [&](int mt, int nt, int v) __attribute__((always_inline)) {
+    const float x = __builtin_fabsf(acc[mt][nt][v]);
+    float least = 0.0f;
+    if (scan) {
+      const int row = (wm * kMT + mt) * 32 + 8 * (v >> 2) + 4 * h + (v & 3), col = TM + (wn * kNT + nt) * 32 + r;
+      if (stat[TM + TN + row]) least += __builtin_bit_cast(float, stat[col]);
+      if (stat[TM + TN + col]) least += __builtin_bit_cast(float, stat[row]);
+      least *= (float)K * kLost;
+    }
+    return x <= __FLT_MAX__ && !(x < least);
+  };
+  uint32_t bad[kMT][kNT] = {};  // per 32×32 block: the lane's sums that do not stand
   if (group == 0) {
     float z = 0.0f;  // stays zero where every sum is finite (x - x is not otherwise)
-    bool low = false;
 #pragma unroll
     for (int i = 0; i < kMT * kNT * 16; ++i) {
       const float x = acc[i / 16 / kNT][i / 16 % kNT][i % 16];
       z += x - x;
-      low |= __builtin_fabsf(x) < least;
     }
-    if (!(z == 0.0f) || low) s_redo = 1;
+    if (scan || early || !(z == 0.0f)) {
+      uint32_t any = 0;
+#pragma unroll
+      for (int i = 0; i < kMT * kNT * 16; ++i) {
+        const int mt = i / 16 / kNT, nt = i / 16 % kNT, v = i % 16;
+        bad[mt][nt] |= (early || !stands(mt, nt, v) ? 1u : 0u) << v;
+        any |= bad[mt][nt];
+      }
+      if (any != 0) s_redo = 1;
+    }
   }
   __syncthreads();
-  if (s_redo) {
-    static_assert(sizeof(Smem) >= 16 * (TM + TN + 64) * sizeof(float), "the fp32 staging fits in the buffers");
-    float* la = reinterpret_cast<float*>(&sms[0]);
-    f32_tile_direct<TM, TN, kMT, kNT, kT>(A, B, M, N, K, m0, n0, t, group == 0, wm, wn, la, la + 16 * (TM + 32), acc);
-  }
-  if (group > 0) return;
+  const bool redo = __builtin_amdgcn_readfirstlane(s_redo) != 0;
   // acc[mt][nt][v] holds C[row][col], row = 8*(v/4) + 4*h + v%4, col = r (within the 32×32 tile).
-  // Only the columns of this tile's own place are stored.
+  // Only the columns of this tile's own place are stored; `again`: only the sums formed again.
   const bool whole = m0 + TM <= M && n0 + TN <= N && n0 == tc.tn * TN;
+  auto store = [&](auto again) __attribute__((always_inline)) {
 #pragma unroll
-  for (int mt = 0; mt < kMT; ++mt)
+    for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      const int col = n0 + (wn * kNT + nt) * 32 + r;
-      const bool cok = col < N && col >= tc.tn * TN;
+      for (int nt = 0; nt < kNT; ++nt) {
+        const int col = n0 + (wn * kNT + nt) * 32 + r;
+        const bool cok = col < N && col >= tc.tn * TN;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = m0 + (wm * kMT + mt) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-        if (whole || (cok && row < M)) C[(size_t)row * N + col] = acc[mt][nt][v];
+        for (int v = 0; v < 16; ++v) {
+          const int row = m0 + (wm * kMT + mt) * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+          if ((whole || (cok && row < M)) && (!again || (bad[mt][nt] >> v & 1u))) C[(size_t)row * N + col] = acc[mt][nt][v];
+        }
       }
-    }
+  };
+  if (group == 0 && !early) store(std::false_type{});
+  if (!redo || group > 0) return;
+  uint32_t need = 0;
+#pragma unroll
+  for (int i = 0; i < kMT * kNT; ++i) need |= __any(bad[i / kNT][i % kNT] != 0) ? 1u << i : 0u;
+  need = (uint32_t)__builtin_amdgcn_readfirstlane((int)need);
+  if (need == 0) return;
+  f32_blocks_direct<kMT, kNT>(A, B, M, N, K, m0 + wm * kMT * 32, n0 + wn * kNT * 32, lane, need, acc);
+  store(std::true_type{});
 }
 
 // Round-to-nearest-even fp32 -> bf16 (quiet NaN kept NaN).

@@ -298,3 +298,46 @@ def test_gemm_f32_error_of_a_float32_sum(ctx, shape):
     a, b = rng.standard_normal((m, k), np.float32), rng.standard_normal((k, n), np.float32)
     ref = a.astype(np.float64) @ b.astype(np.float64)
     assert np.linalg.norm(run_gemm(ctx, a, b) - ref) <= 2.0 ** -24 * (k / 6) ** 0.5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("shape", F32_KERNELS)
+def test_gemm_f32_exceptional_values_stay_in_their_rows_and_columns(ctx, shape):
+    """A sum's arithmetic depends on its row of A and its column of B alone: rows and columns with an
+    infinity, NaN, a value that rounds to infinity in bf16 or values whose pieces are lost leave every
+    other entry's bits as they are."""
+    m, n, k = shape
+    a, b = make_inputs(m, n, k)
+    c = run_gemm(ctx, a, b)
+    odd_a, odd_b = a.copy(), b.copy()
+    rows, cols = [0, 1, 2, 3, m // 2, m - 1], [5, n // 2, n - 1]
+    odd_a[0, 0], odd_a[1, k - 1], odd_a[2, k // 2], odd_a[3, 1] = np.inf, np.nan, -np.inf, 3.4e38
+    odd_a[m // 2] *= np.float32(2.0 ** -126)
+    odd_a[m - 1, 1::2] *= np.float32(2.0 ** -130)
+    odd_b[k - 1, 5], odd_b[:, n // 2], odd_b[0, n - 1] = np.nan, 0.0, -3.4e38
+    got = run_gemm(ctx, odd_a, odd_b)
+    same = np.ones((m, n), bool)
+    same[rows], same[:, cols] = False, False
+    assert np.array_equal(got[same], c[same])
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = odd_a.astype(np.float64) @ odd_b.astype(np.float64)
+        bound = (k + 1) * 2.0 ** -23 * (np.abs(odd_a).astype(np.float64) @ np.abs(odd_b).astype(np.float64)) + 2.0 ** -149 * k
+        fin = np.isfinite(ref) & (np.abs(ref) < 3.4e38)
+        assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.all(np.abs(got[fin] - ref[fin]) <= bound[fin])
+
+
+@pytest.mark.parametrize("shape", F32_KERNELS)
+def test_gemm_f32_values_whose_pieces_are_lost(ctx, shape):
+    """Values near 2^-130 times ones near 2^100: their bf16 pieces would be off by up to 2^-134, a
+    sixteenth of the value. All of A, all of B, one row among ordinary ones, and every third value of it."""
+    m, n, k = shape
+    a, b = make_inputs(m, n, k)
+    small, large = np.float32(2.0 ** -130), np.float32(2.0 ** 100)
+    row, third = a * np.float32(2.0 ** -100), a * np.float32(2.0 ** -100)
+    row[m // 2] = a[m // 2] * small
+    third[m // 2, ::3] = a[m // 2, ::3] * small
+    third[m // 2, 1::3] = third[m // 2, 2::3] = 0
+    for x, y in ((a * small, b * large), (a * large, b * small), (row, b * large), (third, b * large)):
+        got = run_gemm(ctx, x, y)
+        x64, y64 = x.astype(np.float64), y.astype(np.float64)
+        # (the float32 product's error, as in the other tests: each of k additions within one ulp)
+        assert np.all(np.abs(got - x64 @ y64) <= (k + 1) * 2.0 ** -23 * (np.abs(x64) @ np.abs(y64)))
