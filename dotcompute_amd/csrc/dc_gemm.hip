@@ -403,7 +403,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const float* __re
 // and 64×64 with 2×2 waves (64 and 32 KiB, two and four workgroups per CU). KS > 1: KS such wave
 // groups per workgroup, each with LDS buffers of its own, take the k tiles in turn (tile kt goes to
 // group kt mod KS), and their sums are added in group order at the end: more loads in flight for a
-// grid of few tiles. Measured with the dispatch in dc_hip_gemm_bf16: 2000×3000×1000 144 -> 21 us
+// grid of few tiles. Measured (more beside the rule in dc_gemm_route.hpp): 2000×3000×1000 144 -> 21 us
 // (560 TFLOP/s; the kernel it replaces loaded and transposed element by element), 1999×2999×999
 // 31 us; 8192^3 0.84 ms (1300 TFLOP/s), as before. The big tile is bound by the matrix cores' power
 // limit and its tile barriers, the small ones by the latency of one tile's loads per barrier.
@@ -453,9 +453,9 @@ typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
 // 8 bf16 at the alignment of one (the unaligned 16-byte load)
 typedef unsigned short u16x8_any __attribute__((ext_vector_type(8), aligned(2)));
 
-// Buffer range of the kDma loader: the host keeps every byte offset below it, so a lane that must
-// load zeros asks for kPastRange, whatever the uniform offset added to it.
-constexpr int32_t kDmaRange = 0x7FFFFFFF;
+// Buffer range of the kDma loader: the host keeps every byte offset below it (dc_gemm_route.hpp), so a
+// lane that must load zeros asks for kPastRange, whatever the uniform offset added to it.
+constexpr int32_t kDmaRange = dc::kBf16DmaRange;
 constexpr uint32_t kPastRange = 0x80000000u;
 
 // Issues the direct-to-LDS loads of the k tile at k0 (klim = k rows left from there) for the panels
@@ -1338,34 +1338,17 @@ DC_HIP_API int32_t dc_hip_gemm_bf16(dc_hip_ctx* ctx, const uint16_t* a, const ui
   if (k == 0) return dc::zero_async(ctx, c, (size_t)(m * n) * sizeof(float));
   const unsigned short* A = reinterpret_cast<const unsigned short*>(a);
   const unsigned short* B = reinterpret_cast<const unsigned short*>(b);
-  // 16-byte rows, and every byte offset of the panels (256 rows of A; B's rows, with up to four k
-  // tiles past the last) inside the buffer range: the direct-to-LDS loader
-  const bool dma = n % 8 == 0 && k % 8 == 0 && dc::aligned16(a) && dc::aligned16(b) &&
-                   (k + 4 * kBK2) * 256 * 2 < (int64_t)kDmaRange && (k + 4 * kBK2) * n * 2 < (int64_t)kDmaRange;
-  // The widest tile that still gives the chip enough workgroups; then, where even the small tiles
-  // leave CUs idle, a k dimension split over the wave groups of a workgroup. Measured (us, direct-to-LDS
-  // loader, tiles 256 / 128 / 64; "x2", "x4": that many k groups):
-  //   3072x3072x1024 (144 tiles of 256): 27.5 / 32.6 / 33.8;  2048x8192x512 (256): 24.1 / 26.5 / 31.4
-  //   2000x3000x1000 (96 tiles of 256, 384 of 128): 29.0 / 21.2 / 28.8
-  //   2048^3 (256 of 128): 45.2 / 28.2 (x2 23.7) / 27.3;  1536^3 (144): 34.6 / 20.3 (x2 17.5) / 15.2
-  //   256x8192x8192 (512 of 64): 151 / 80 / 61, x2 51.8, x4 66;  1024^3 (256 of 64): 7.4, x2 6.6, x4 6.7
-  //   64x8192x8192 (128 of 64): 61, x2 43, x4 36;  512x512x4096 (64 of 64): 32, x2 24, x4 20
-  //   512^3: 4.6, x2 4.4, x4 4.9
-  // Register loader (128 / 64): 2047^3 42 / 52, 1535^3 33 / 29, 1023^3 21 / 12.4 (x4 11.0),
-  // 511x511x4095 61 / 48 (x4 32).
-  const int64_t cus = std::max(1, ctx->cu_count);
-  auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
-  if (dma) {
-    if (2 * tiles(256) > cus) launch_bf16<256, 256, 2, 4, 1, true>(ctx, A, B, c, m, n, k);
-    else if (tiles(128) > cus) launch_bf16<128, 128, 2, 2, 1, true>(ctx, A, B, c, m, n, k);
-    else if (4 * tiles(128) > 3 * cus) launch_bf16<128, 128, 2, 2, 2, true>(ctx, A, B, c, m, n, k);
-    else if (tiles(64) > 2 * cus || k < 512) launch_bf16<64, 64, 2, 2, 1, true>(ctx, A, B, c, m, n, k);
-    else if (2 * tiles(64) > cus || k < 2048) launch_bf16<64, 64, 2, 2, 2, true>(ctx, A, B, c, m, n, k);
-    else launch_bf16<64, 64, 2, 2, 4, true>(ctx, A, B, c, m, n, k);
-  } else {
-    if (n >= 128 && 4 * tiles(128) > 3 * cus) launch_bf16<128, 128, 2, 2, 1, false>(ctx, A, B, c, m, n, k);
-    else if (tiles(64) > cus || k < 1000) launch_bf16<64, 64, 2, 2, 1, false>(ctx, A, B, c, m, n, k);
-    else launch_bf16<64, 64, 2, 2, 4, false>(ctx, A, B, c, m, n, k);
+  using dc::Bf16Gemm;
+  switch (dc::bf16_gemm_kernel(m, n, k, dc::aligned16(a) && dc::aligned16(b), std::max(1, ctx->cu_count))) {
+    case Bf16Gemm::kDma256: launch_bf16<256, 256, 2, 4, 1, true>(ctx, A, B, c, m, n, k); break;
+    case Bf16Gemm::kDma128: launch_bf16<128, 128, 2, 2, 1, true>(ctx, A, B, c, m, n, k); break;
+    case Bf16Gemm::kDma128x2: launch_bf16<128, 128, 2, 2, 2, true>(ctx, A, B, c, m, n, k); break;
+    case Bf16Gemm::kDma64: launch_bf16<64, 64, 2, 2, 1, true>(ctx, A, B, c, m, n, k); break;
+    case Bf16Gemm::kDma64x2: launch_bf16<64, 64, 2, 2, 2, true>(ctx, A, B, c, m, n, k); break;
+    case Bf16Gemm::kDma64x4: launch_bf16<64, 64, 2, 2, 4, true>(ctx, A, B, c, m, n, k); break;
+    case Bf16Gemm::kReg128: launch_bf16<128, 128, 2, 2, 1, false>(ctx, A, B, c, m, n, k); break;
+    case Bf16Gemm::kReg64: launch_bf16<64, 64, 2, 2, 1, false>(ctx, A, B, c, m, n, k); break;
+    case Bf16Gemm::kReg64x4: launch_bf16<64, 64, 2, 2, 4, false>(ctx, A, B, c, m, n, k); break;
   }
   return dc::last_launch_status();
 }

@@ -51,4 +51,50 @@ inline F32Gemm f32_gemm_kernel(int64_t m, int64_t n, int64_t k, bool aligned16, 
   return k < 1536 ? F32Gemm::kSplit64x2 : F32Gemm::kSplit64x4;
 }
 
+// bf16: "Dma": direct-to-LDS loads, by tile (square) and k groups; "Reg": loads through registers.
+enum class Bf16Gemm { kDma256, kDma128, kDma128x2, kDma64, kDma64x2, kDma64x4, kReg128, kReg64, kReg64x4 };
+
+// Bytes that a direct-to-LDS load of the bf16 kernels can be away from its panel's first.
+constexpr int32_t kBf16DmaRange = INT32_MAX;
+
+// Measured, us (256 CUs; tiles 256 / 128 / 64, "x2", "x4": that many k groups):
+//   3072x3072x1024 (144 tiles of 256): 27.5 / 32.6 / 33.8;  2048x8192x512 (256): 24.1 / 26.5 / 31.4
+//   4352x4096x1024 (272): 57.4 / 52.0 / 60.9;  4608x4608x1024 (324): 60.4 / 56.8 / 73.7
+//   5120x5120x1024 (400): 63.1 / 69.7 / 86.2;  6144x6144x1024 (576): 94.7 / 93.8 / 121.8
+//   8192x8192x64: 54.4 / 46.3 / 46.1;  4096x4096x64: 14.0 / 14.5 / 15.5;  2048x2048x64: 9.6 / 6.8 / 6.0
+//   8192x8192x128: 61.7 / 58.6 / 57.5;  4096x4096x128: 15.8 / 16.2 / 17.3;  4352x4096x64: 20.1 / 17.1 / 15.9
+//   2000x3000x1000 (96 tiles of 256, 384 of 128): 29.0 / 21.2 / 28.8
+//   2048^3 (256 of 128): 45.2 / 28.2 (x2 23.7) / 27.3;  1536^3 (144): 34.6 / 20.3 (x2 17.5) / 15.2
+//   256x8192x8192 (512 of 64): 151 / 80 / 61, x2 51.8, x4 66;  1024^3 (256 of 64): 7.4, x2 6.6, x4 6.7
+//   64x8192x8192 (128 of 64): 61, x2 43, x4 36;  512x512x4096 (64 of 64): 32, x2 24, x4 20
+//   512^3: 4.6, x2 4.4, x4 4.9
+// Register loader (128 / 64): 2047^3 42 / 52, 1535^3 33 / 29, 1023^3 21 / 12.4 (x4 11.0),
+// 511x511x4095 61 / 48 (x4 32).
+inline Bf16Gemm bf16_gemm_kernel(int64_t m, int64_t n, int64_t k, bool aligned16, int64_t cus) {
+  auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
+  const int64_t t256 = tiles(256), t128 = tiles(128), t64 = tiles(64);
+  if (n % 8 == 0 && k % 8 == 0 && aligned16) {
+    // The widest tile that still gives the chip enough workgroups, but where a second round of the
+    // 256-tiles would be mostly empty or k is too short for them; then, where even the small tiles leave
+    // CUs idle, a k dimension split over the wave groups of a workgroup.
+    struct Choice {
+      Bf16Gemm kernel;
+      int64_t tile, groups;
+    } c;
+    const bool brief = (k <= 64 && (t256 > cus || 4 * t256 <= 3 * cus)) || (k <= 128 && t256 > 2 * cus);
+    if (2 * t256 > cus && (t256 <= cus || 10 * t256 > 13 * cus) && !brief) c = {Bf16Gemm::kDma256, 256, 1};
+    else if (t128 > cus && !brief) c = {Bf16Gemm::kDma128, 128, 1};
+    else if (4 * t128 > 3 * cus && k > 128) c = {Bf16Gemm::kDma128x2, 128, 2};
+    else if (t64 > 2 * cus || k < 512) c = {Bf16Gemm::kDma64, 64, 1};
+    else if (2 * t64 > cus || k < 2048) c = {Bf16Gemm::kDma64x2, 64, 2};
+    else c = {Bf16Gemm::kDma64x4, 64, 4};
+    // Every byte offset inside the buffer range: of the tile's rows of A, and of B's rows with those past
+    // the last that the groups' k tiles ask for (zeros). Larger shapes go through registers.
+    const int64_t rows = (k + 64 * c.groups - 1) / (64 * c.groups) * (64 * c.groups);
+    if (c.tile * k * 2 < kBf16DmaRange && rows * n * 2 < kBf16DmaRange) return c.kernel;
+  }
+  if (n >= 128 && 4 * t128 > 3 * cus) return Bf16Gemm::kReg128;
+  return t64 > cus || k < 1000 ? Bf16Gemm::kReg64 : Bf16Gemm::kReg64x4;
+}
+
 }  // namespace dc

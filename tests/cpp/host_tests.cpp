@@ -211,6 +211,34 @@ std::shared_ptr<Backends::Hip::HipAccelerator> Gpu() {
 
 // ============================== CPU: fusion planner ==============================================
 
+// The bf16 shapes of tests/test_gpu_gemm.py, each rule's edges, and the buffer range: a shape keeps the
+// direct-to-LDS loads while the rows that its own kernel asks for are inside it.
+TEST_CPU(GemmBf16_EachShapeTakesItsKernel) {
+  using dc::Bf16Gemm;
+  struct Row {
+    int64_t m, n, k;
+    Bf16Gemm want;
+  };
+  const Row rows[] = {
+      {2824, 3080, 72, Bf16Gemm::kDma256}, {4104, 4360, 136, Bf16Gemm::kDma128}, {2200, 2056, 200, Bf16Gemm::kDma128},
+      {1800, 1912, 136, Bf16Gemm::kDma128x2}, {200, 264, 200, Bf16Gemm::kDma64}, {2824, 3080, 64, Bf16Gemm::kDma64},
+      {4096, 4096, 64, Bf16Gemm::kDma256},
+      {456, 520, 520, Bf16Gemm::kDma64x2}, {72, 136, 2120, Bf16Gemm::kDma64x4}, {1799, 1911, 137, Bf16Gemm::kReg128},
+      {63, 65, 129, Bf16Gemm::kReg64}, {300, 50, 70, Bf16Gemm::kReg64}, {129, 131, 1001, Bf16Gemm::kReg64x4},
+      // B of 501 * 256 columns and 8192 rows is 2.101e9 bytes; 8256 rows of 130056 columns pass 2^31
+      {8, 128256, 8192, Bf16Gemm::kDma256}, {8, 130048, 8200, Bf16Gemm::kDma256}, {8, 130056, 8200, Bf16Gemm::kReg128},
+      {8, 131064, 8192, Bf16Gemm::kDma256}, {8, 131072, 8192, Bf16Gemm::kReg128},
+      // four groups' k tiles: 2^24 rows of 64 columns end at 2^31 with the last; 256 rows less do not
+      {8, 64, (1 << 24), Bf16Gemm::kReg64x4}, {8, 64, (1 << 24) - 256, Bf16Gemm::kDma64x4},
+      {8, 64, (1 << 24) - 248, Bf16Gemm::kReg64x4},
+      // 256 rows of A
+      {40000, 128, 4194296, Bf16Gemm::kDma256}, {40000, 256, 4194304, Bf16Gemm::kReg128}};
+  for (const Row& r : rows)
+    if (dc::bf16_gemm_kernel(r.m, r.n, r.k, true, 256) != r.want)
+      throw dctest::Failure(std::to_string(r.m) + "x" + std::to_string(r.n) + "x" + std::to_string(r.k));
+  CHECK(dc::bf16_gemm_kernel(2824, 3080, 72, false, 256) == Bf16Gemm::kReg128);
+}
+
 // The shapes of tests/test_gpu_gemm.py that are there for one kernel each, and each rule's edges.
 TEST_CPU(GemmF32_EachShapeTakesItsKernel) {
   using dc::F32Gemm;

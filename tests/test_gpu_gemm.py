@@ -172,10 +172,10 @@ def test_convert_f32_to_bf16_bit_exact(ctx):
 
 
 # One shape or two per tile choice of the bf16 dispatch (on 256 CUs), each with ragged rows, columns
-# and a last k tile that is not whole. 16-byte rows: 256-tiles, 128-tiles, 128-tiles with two k groups,
-# 64-tiles with one, two and four; other rows: 128-tiles, 64-tiles with one and four k groups,
-# fewer columns than a tile.
-@pytest.mark.parametrize("shape", [(2824, 3080, 72), (2200, 2056, 200), (1800, 1912, 136), (200, 264, 200), (8, 8, 8),
+# and a last k tile that is not whole. 16-byte rows: 256-tiles, 128-tiles (two), 128-tiles with two k
+# groups, 64-tiles with one, two and four; other rows: 128-tiles, 64-tiles with one and four k groups,
+# fewer columns than a tile. (host_tests.cpp checks that each shape takes the kernel it is here for.)
+@pytest.mark.parametrize("shape", [(2824, 3080, 72), (4104, 4360, 136), (2200, 2056, 200), (1800, 1912, 136), (200, 264, 200), (8, 8, 8),
                                    (456, 520, 520), (72, 136, 2120), (1799, 1911, 137), (63, 65, 129), (300, 50, 70),
                                    (129, 131, 1001), (70, 9, 64)])
 def test_gemm_bf16_ragged_tiles(ctx, shape):
@@ -341,3 +341,25 @@ def test_gemm_f32_values_whose_pieces_are_lost(ctx, shape):
         x64, y64 = x.astype(np.float64), y.astype(np.float64)
         # (the float32 product's error, as in the other tests: each of k additions within one ulp)
         assert np.all(np.abs(got - x64 @ y64) <= (k + 1) * 2.0 ** -23 * (np.abs(x64) @ np.abs(y64)))
+
+
+@pytest.mark.slow
+@pytest.mark.parametrize("shape", [(8, 128256, 8192), (8, 130048, 8200), (8, 130056, 8200)])
+def test_gemm_bf16_b_of_almost_two_gib(ctx, shape):
+    """B's byte offsets up to the end of the direct-to-LDS loads' buffer range, and just past it."""
+    m, n, k = shape
+    rng = np.random.default_rng(n)
+    a = oracle.f32_to_bf16(rng.uniform(-1, 1, m * k).astype(np.float32)).reshape(m, k)
+    part = oracle.f32_to_bf16(rng.uniform(-1, 1, 1000003).astype(np.float32))  # (a prime: no two rows alike)
+    b = np.resize(part, n * k).reshape(k, n)
+    da, db, c = ctx.to_device(a), ctx.to_device(b), ctx.empty((m, n), np.float32)
+    ctx.gemm_bf16(da, db, c, m, n, k)
+    ctx.synchronize()
+    got = c.to_host()
+    for x in (da, db, c):
+        ctx.free(x)
+    cols = np.unique(np.concatenate([rng.integers(0, n, 150), np.arange(n - 10, n), np.arange(10)]))
+    a64 = oracle.bf16_to_f32(a).reshape(m, k).astype(np.float64)
+    b64 = oracle.bf16_to_f32(np.ascontiguousarray(b[:, cols])).reshape(k, -1).astype(np.float64)
+    # products of bf16 values are exact in float32; k additions, each within one float32 ulp
+    assert np.all(np.abs(got[:, cols] - a64 @ b64) <= k * 2.0 ** -23 * (np.abs(a64) @ np.abs(b64)))
