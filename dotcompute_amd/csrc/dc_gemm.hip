@@ -46,12 +46,16 @@ constexpr int kThreads = 256;
 constexpr int kGroupM = 8;
 
 struct TileCoord {
-  int tm, tn;
+  int tm, tn;  // tm < 0: none (past the last tile, in a grid of more than one row)
 };
 
 __device__ inline TileCoord map_tile(int tiles_m, int tiles_n) {
   const int total = tiles_m * tiles_n;
   int b = blockIdx.x;
+  if (blockIdx.y != 0) {  // (dc::gemm_grid)
+    b += (int)(blockIdx.y * gridDim.x);
+    if (b >= total) return TileCoord{-1, 0};
+  }
   int t = (total % 8 == 0) ? (b % 8) * (total / 8) + b / 8 : b;
   const int group = kGroupM * tiles_n;
   const int g = t / group;
@@ -128,6 +132,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_dma_kernel(const float* 
   __shared__ __align__(16) float lds_a0[T * kBKd], lds_a1[T * kBKd], lds_b0[kBKd * T], lds_b1[kBKd * T];
   const F32DmaSmem<T> sm{{lds_a0, lds_a1}, {lds_b0, lds_b1}};
   const TileCoord tc = map_tile(tiles_m, tiles_n);
+  if (tc.tm < 0) return;
   const int m0 = tc.tm * T, n0 = tc.tn * T;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -329,6 +334,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const float* __re
   constexpr int kW = T / 2, kMT = T / 64;  // wave tile edge, MFMA tiles per wave edge
   __shared__ F32Smem<BK, T> sm;
   const TileCoord tc = map_tile(tiles_m, tiles_n);
+  if (tc.tm < 0) return;
   const int m0 = tc.tm * T, n0 = tc.tn * T;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -491,6 +497,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
   using Smem = Bf16Smem<TM, TN>;
   __shared__ __align__(16) Smem sms[KS];
   const TileCoord tc = map_tile(tiles_m, tiles_n);
+  if (tc.tm < 0) return;
   const int m0 = tc.tm * TM;
   // (register loader: the last tile ends at N where N holds a whole tile)
   const int n0 = kDma || N < TN ? tc.tn * TN : min(tc.tn * TN, N - TN);
@@ -933,6 +940,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
   __shared__ int s_redo, s_tiny, s_low;
   __shared__ uint32_t s_seen, s_big;
   const TileCoord tc = map_tile(tiles_m, tiles_n);
+  if (tc.tm < 0) return;
   const int m0 = tc.tm * TM;
   const int n0 = min(tc.tn * TN, N - TN);  // the last tile ends at N (N >= TN, by the host)
   const int tid = threadIdx.x, lane = tid & 63, gwave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1277,18 +1285,25 @@ __global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float* __restric
 
 constexpr int kBKf32 = 32;
 
+dim3 tile_grid(int tiles_m, int tiles_n, int threads) {
+  const dc::GemmGrid g = dc::gemm_grid((int64_t)tiles_m * tiles_n, threads);
+  return dim3((unsigned)g.x, (unsigned)g.rows);
+}
+
 template <int TM, int TN, int WM, int WN, int KS, bool kDma>
 void launch_bf16(dc_hip_ctx* ctx, const unsigned short* a, const unsigned short* b, float* c, int64_t m, int64_t n,
                  int64_t k) {
+  constexpr int kThr = 64 * WM * WN * KS;
   const int tiles_m = (int)((m + TM - 1) / TM), tiles_n = (int)((n + TN - 1) / TN);
-  gemm_bf16_kernel<TM, TN, WM, WN, KS, kDma><<<(unsigned)(tiles_m * tiles_n), 64 * WM * WN * KS, 0, ctx->stream>>>(
+  gemm_bf16_kernel<TM, TN, WM, WN, KS, kDma><<<tile_grid(tiles_m, tiles_n, kThr), kThr, 0, ctx->stream>>>(
       a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
 }
 
 template <int TM, int TN, int WM, int WN, int KS, int D>
 void launch_split(dc_hip_ctx* ctx, const float* a, const float* b, float* c, int64_t m, int64_t n, int64_t k) {
+  constexpr int kThr = 64 * WM * WN * KS;
   const int tiles_m = (int)((m + TM - 1) / TM), tiles_n = (int)((n + TN - 1) / TN);
-  gemm_f32_split_kernel<TM, TN, WM, WN, KS, D><<<(unsigned)(tiles_m * tiles_n), 64 * WM * WN * KS, 0, ctx->stream>>>(
+  gemm_f32_split_kernel<TM, TN, WM, WN, KS, D><<<tile_grid(tiles_m, tiles_n, kThr), kThr, 0, ctx->stream>>>(
       a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
 }
 
@@ -1312,11 +1327,11 @@ DC_HIP_API int32_t dc_hip_gemm_f32(dc_hip_ctx* ctx, const float* a, const float*
   const int tiles_m = (int)((m + 63) / 64), tiles_n = (int)((n + 63) / 64);
   switch (dc::f32_gemm_kernel(m, n, k, dc::aligned16(a) && dc::aligned16(b), std::max(1, ctx->cu_count))) {
     case dc::F32Gemm::kDma64:
-      gemm_f32_dma_kernel<64><<<(unsigned)(tiles_m * tiles_n), kThreads, 0, ctx->stream>>>(a, b, c, (int)m, (int)n, (int)k,
-                                                                                         tiles_m, tiles_n);
+      gemm_f32_dma_kernel<64><<<tile_grid(tiles_m, tiles_n, kThreads), kThreads, 0, ctx->stream>>>(
+          a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
       break;
     case dc::F32Gemm::kChecked64:
-      gemm_f32_kernel<kBKf32, true, 64><<<(unsigned)(tiles_m * tiles_n), kThreads, 0, ctx->stream>>>(
+      gemm_f32_kernel<kBKf32, true, 64><<<tile_grid(tiles_m, tiles_n, kThreads), kThreads, 0, ctx->stream>>>(
           a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
       break;
     case dc::F32Gemm::kSplit256x128: launch_split<256, 128, 4, 2, 1, 1>(ctx, a, b, c, m, n, k); break;

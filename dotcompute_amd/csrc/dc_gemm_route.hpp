@@ -6,6 +6,16 @@
 
 namespace dc {
 
+// The grid of `tiles` workgroups: rows of `x` of them, more than one row where a single one would have
+// more work items than a launch takes in a dimension (2^32 - 1); the last row may be partly empty.
+struct GemmGrid {
+  int64_t x, rows;
+};
+inline GemmGrid gemm_grid(int64_t tiles, int64_t threads) {
+  const int64_t most = (int64_t)UINT32_MAX / threads, rows = (tiles + most - 1) / most;
+  return {(tiles + rows - 1) / rows, rows};
+}
+
 // fp32: "Split": the bf16 matrix cores, by tile (rows x columns) and k groups; the others the fp32
 // instructions (Dma64: direct-to-LDS loads of full 64-tiles; Checked64: any shape).
 enum class F32Gemm { kDma64, kChecked64, kSplit256x128, kSplit128, kSplit128x2, kSplit64, kSplit64x2, kSplit64x4 };

@@ -211,6 +211,16 @@ std::shared_ptr<Backends::Hip::HipAccelerator> Gpu() {
 
 // ============================== CPU: fusion planner ==============================================
 
+TEST_CPU(GemmGrid_StaysWithinALaunch) {
+  for (int64_t threads : {256, 512, 1024})
+    for (int64_t tiles : {int64_t(1), int64_t(UINT32_MAX) / threads, int64_t(UINT32_MAX) / threads + 1, int64_t(1) << 24,
+                          (int64_t(1) << 24) + 1, int64_t(27000000)}) {
+      const dc::GemmGrid g = dc::gemm_grid(tiles, threads);
+      CHECK(g.x * threads <= int64_t(UINT32_MAX) && g.x * g.rows >= tiles && g.x * (g.rows - 1) < tiles);
+      CHECK((g.rows == 1) == (tiles * threads <= int64_t(UINT32_MAX)));
+    }
+}
+
 // The bf16 shapes of tests/test_gpu_gemm.py, each rule's edges, and the buffer range: a shape keeps the
 // direct-to-LDS loads while the rows that its own kernel asks for are inside it.
 TEST_CPU(GemmBf16_EachShapeTakesItsKernel) {

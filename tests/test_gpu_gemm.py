@@ -363,3 +363,22 @@ def test_gemm_bf16_b_of_almost_two_gib(ctx, shape):
     b64 = oracle.bf16_to_f32(np.ascontiguousarray(b[:, cols])).reshape(k, -1).astype(np.float64)
     # products of bf16 values are exact in float32; k additions, each within one float32 ulp
     assert np.all(np.abs(got[:, cols] - a64 @ b64) <= k * 2.0 ** -23 * (np.abs(a64) @ np.abs(b64)))
+
+
+@pytest.mark.slow
+@pytest.mark.parametrize("kind,m,n", [("f32", 2 ** 30 - 1, 1), ("f32", 1, 2 ** 30 - 1), ("bf16", 2 ** 30 - 1, 1)])
+def test_gemm_longest_vectors(ctx, kind, m, n):
+    """The largest m and n that the entries take: 2^24 tiles of 64, more work items than one row of a grid."""
+    part = np.random.default_rng(1).integers(-100, 100, 1000003).astype(np.float32)  # exact in bf16
+    long = np.resize(part if kind == "f32" else oracle.f32_to_bf16(part), max(m, n))
+    other = np.full(1, 2.0, np.float32)
+    dl, do = ctx.to_device(long), ctx.to_device(other if kind == "f32" else oracle.f32_to_bf16(other))
+    c = ctx.empty(m * n, np.float32)
+    (ctx.gemm_f32 if kind == "f32" else ctx.gemm_bf16)(*((dl, do) if m > n else (do, dl)), c, m, n, 1)
+    ctx.synchronize()
+    got = c.to_host()
+    for x in (dl, do, c):
+        ctx.free(x)
+    whole = got[: got.size // part.size * part.size].reshape(-1, part.size)
+    assert np.array_equal(whole[0], 2 * part) and (whole == whole[0]).all()
+    assert np.array_equal(got[whole.size:], 2 * part[:got.size - whole.size])
