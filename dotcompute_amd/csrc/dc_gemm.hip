@@ -7,7 +7,7 @@
 // Kernels, by the shapes that take them:
 //   - gemm_f32_split_kernel<TM, TN, ...>: fp32, by eight bf16 products per fp32 product; 256×128,
 //     128×128 or 64×64 macro tiles (the rule and its measurements: dc_gemm_route.hpp).
-//   - gemm_f32_dma_kernel<64>: fp32 full 64-tiles with a short k or few of them, on the fp32
+//   - gemm_f32_dma_kernel: fp32 full 64-tiles with a short k or few of them, on the fp32
 //     instructions: direct-to-LDS loads, double-buffered LDS, 4 waves of 32×32.
 //   - gemm_f32_kernel: the fp32 shapes left (fewer than 64 columns, at most 16 rows of B),
 //     bounds-checked 64×64 tiles on the fp32 instructions.
@@ -66,28 +66,27 @@ __device__ inline TileCoord map_tile(int tiles_m, int tiles_n) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp32, full tiles (m, n multiples of T, k a multiple of 32): direct-to-LDS loads, no staging
-// registers and no transposing LDS stores. Launched with T = 64 for a short k or few tiles (1024^3:
-// 18.9 us; see dc_gemm_route.hpp).
-//   A tile [T rows][32 k] (128 B rows, unpadded): the 16-byte k-quad q of row R sits in slot
+// fp32, full 64×64 tiles (m, n multiples of 64, k of 32): direct-to-LDS loads, no staging registers and
+// no transposing LDS stores. For a short k or few tiles (1024^3: 18.9 us; see dc_gemm_route.hpp).
+//   A tile [64 rows][32 k] (128 B rows, unpadded): the 16-byte k-quad q of row R sits in slot
 //   q ^ ((R >> 1) & 7), so a fragment read (16 lanes = rows R0..R0+15 at one quad) touches 16
 //   distinct 16-byte bank groups.
-//   B tile [32 k][T n] in its natural row-major layout: the n-quad Q of k-row k sits at quad
+//   B tile [32 k][64 n] in its natural row-major layout: the n-quad Q of k-row k sits at quad
 //   Q ^ (8·((k >> 3) & 1)). Lane (r, h) of MFMA step kk reads B[ks + 8h + kk][n = r] with a 4-byte
 //   LDS load: the h = 0 and h = 1 halves read rows 8 apart and land in opposite 128-byte halves of
 //   the bank window.
 // A wave's direct-to-LDS load writes 1 KiB (lane L -> bytes 16·L): the swizzles are applied on
 // the global side (each lane fetches the quad that belongs in its slot).
-// Pipeline as in the bf16 large-tile kernel: step 0 (k 0..15) runs its MFMAs with step 1's
-// fragment reads between them; then the tile's one barrier (which also waits for tile kt+1's
-// loads, issued a tile earlier); the loads of tile kt+2 go out into the buffer tile kt finished
-// with, and step 1's MFMAs run with tile kt+1's step-0 fragment reads between them.
+// Pipeline as in the bf16 kernel: step 0 (k 0..15) runs its MFMAs with step 1's fragment reads
+// between them; then the tile's one barrier (which also waits for tile kt+1's loads, issued a tile
+// earlier); the loads of tile kt+2 go out into the buffer tile kt finished with, and step 1's
+// MFMAs run with tile kt+1's step-0 fragment reads between them.
 // ---------------------------------------------------------------------------------------------
-constexpr int kBKd = 32;
+constexpr int kT32 = 64;   // macro tile of the kernels on the fp32 instructions: 2×2 waves of 32×32
+constexpr int kBK32 = 32;  // their k slice
 
 // One LDS buffer per (operand, stage) as a separate __shared__ object, so the compiler can tell that
 // loads into one stage's buffers do not alias reads of the other's (and need no wait before them).
-template <int T>
 struct F32DmaSmem {
   float* a[2];
   float* b[2];
@@ -102,106 +101,85 @@ __device__ inline void dma_barrier() {
   __syncthreads();
 }
 
-template <int T, int BUF>
-__device__ inline void f32_tile_to_lds(const F32DmaSmem<T>& sm, __amdgpu_buffer_rsrc_t ra, const float* __restrict__ B, int N,
-                                       int K, int n0, int k0, int wave, uint32_t avoff, const uint32_t (&bvoff)[T / 32]) {
-  // A: T/8 blocks of 8 rows; wave w issues blocks w, w + 4, ...
+template <int BUF>
+__device__ inline void f32_tile_to_lds(const F32DmaSmem& sm, __amdgpu_buffer_rsrc_t ra, const float* __restrict__ B, int N,
+                                       int K, int n0, int k0, int wave, uint32_t avoff, const uint32_t (&bvoff)[2]) {
+  // A: 8 blocks of 8 rows; wave w issues blocks w and w + 4
 #pragma unroll
-  for (int i = 0; i < T / 32; ++i) {
+  for (int i = 0; i < 2; ++i) {
     const int row0 = 8 * (4 * i + wave);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(sm.a[BUF] + row0 * kBKd), 16, avoff,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(sm.a[BUF] + row0 * kBK32), 16, avoff,
                                              (row0 * K + k0) * (int)sizeof(float), 0, 0);
   }
-  // B: T/8 blocks of 256/T k-rows (this k slice only, as its own buffer range)
-  const auto rb = dc::range_rsrc(B + (size_t)k0 * N + n0, ((kBKd - 1) * N + T) * (int)sizeof(float));
-  constexpr int kRowsPerBlock = 256 / T;
+  // B: 8 blocks of 4 k-rows (this k slice only, as its own buffer range)
+  const auto rb = dc::range_rsrc(B + (size_t)k0 * N + n0, ((kBK32 - 1) * N + kT32) * (int)sizeof(float));
 #pragma unroll
-  for (int i = 0; i < T / 32; ++i) {
-    const int krow0 = kRowsPerBlock * (4 * i + wave);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(sm.b[BUF] + krow0 * T), 16, bvoff[i],
+  for (int i = 0; i < 2; ++i) {
+    const int krow0 = 4 * (4 * i + wave);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(sm.b[BUF] + krow0 * kT32), 16, bvoff[i],
                                              krow0 * N * (int)sizeof(float), 0, 0);
   }
 }
 
-template <int T>
 __global__ __launch_bounds__(kThreads, 2) void gemm_f32_dma_kernel(const float* __restrict__ A,
                                                                    const float* __restrict__ B, float* __restrict__ C,
-                                                                   int M, int N, int K, int tiles_m, int tiles_n) {
-  constexpr int kW = T / 2, kMT = T / 64;  // wave tile edge, MFMA tiles per wave edge
-  constexpr int kQuads = T / 4;            // n-quads per B row
-  __shared__ __align__(16) float lds_a0[T * kBKd], lds_a1[T * kBKd], lds_b0[kBKd * T], lds_b1[kBKd * T];
-  const F32DmaSmem<T> sm{{lds_a0, lds_a1}, {lds_b0, lds_b1}};
+                                                                   int N, int K, int tiles_m, int tiles_n) {
+  constexpr int kQuads = kT32 / 4;  // n-quads per B row
+  __shared__ __align__(16) float lds_a0[kT32 * kBK32], lds_a1[kT32 * kBK32], lds_b0[kBK32 * kT32], lds_b1[kBK32 * kT32];
+  const F32DmaSmem sm{{lds_a0, lds_a1}, {lds_b0, lds_b1}};
   const TileCoord tc = map_tile(tiles_m, tiles_n);
   if (tc.tm < 0) return;
-  const int m0 = tc.tm * T, n0 = tc.tn * T;
+  const int m0 = tc.tm * kT32, n0 = tc.tn * kT32;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int r = lane & 31, h = lane >> 5;
 
-  // load side: A panel as a buffer range (T rows of K floats < 2 GiB, checked by the host)
-  const auto ra = dc::range_rsrc(A + (size_t)m0 * K, T * K * (int)sizeof(float));
+  // load side: A panel as a buffer range (64 rows of K floats < 2 GiB, checked by the host)
+  const auto ra = dc::range_rsrc(A + (size_t)m0 * K, kT32 * K * (int)sizeof(float));
   // A block 4i + w holds rows 8(4i + w) + L/8: (row >> 1) & 7 = (4·(w & 1) + L/16) & 7
   const uint32_t avoff =
       (uint32_t)(((lane >> 3) * K + 4 * ((lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7))) * (int)sizeof(float));
-  uint32_t bvoff[T / 32];
+  uint32_t bvoff[2];
 #pragma unroll
-  for (int i = 0; i < T / 32; ++i) {
-    const int kr = lane / kQuads;                        // k-row within the block
-    const int k = (256 / T) * (4 * i + wave) + kr;       // k-row within the slice
+  for (int i = 0; i < 2; ++i) {
+    const int kr = lane / kQuads;            // k-row within the block
+    const int k = 4 * (4 * i + wave) + kr;   // k-row within the slice
     const int q = (lane % kQuads) ^ (8 * ((k >> 3) & 1));
     bvoff[i] = (uint32_t)((kr * N + 4 * q) * (int)sizeof(float));
   }
 
-  f32x16 acc[kMT][kMT];
+  f32x16 acc;
 #pragma unroll
-  for (int i = 0; i < kMT; ++i)
-#pragma unroll
-    for (int j = 0; j < kMT; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
 
-  const int kt_count = K / kBKd;
-  f32_tile_to_lds<T, 0>(sm, ra, B, N, K, n0, 0, wave, avoff, bvoff);
+  const int kt_count = K / kBK32;
+  f32_tile_to_lds<0>(sm, ra, B, N, K, n0, 0, wave, avoff, bvoff);
   dma_barrier();
-  if (kt_count > 1) f32_tile_to_lds<T, 1>(sm, ra, B, N, K, n0, kBKd, wave, avoff, bvoff);
+  if (kt_count > 1) f32_tile_to_lds<1>(sm, ra, B, N, K, n0, kBK32, wave, avoff, bvoff);
 
-  // Fragments of one 16-wide k step: A quads (2 per MFMA tile row block), B scalars (8 per column block).
-  const int aswz = (r >> 1) & 7;
-  auto read_frags = [&](auto BUF, int ks, dc::f32x4 (&a)[kMT][2], float (&b)[kMT][8]) __attribute__((always_inline)) {
+  // Fragments of one 16-wide k step: two A quads, 8 B scalars.
+  const int arow = wm * 32 + r, aswz = (r >> 1) & 7, n = wn * 32 + r;
+  auto read_frags = [&](auto BUF, int ks, dc::f32x4 (&a)[2], float (&b)[8]) __attribute__((always_inline)) {
     constexpr int kB = decltype(BUF)::value;
 #pragma unroll
-    for (int mt = 0; mt < kMT; ++mt)
+    for (int j = 0; j < 2; ++j)
+      a[j] = *reinterpret_cast<const dc::f32x4*>(&(kB ? lds_a1 : lds_a0)[arow * kBK32 + 4 * ((ks / 4 + 2 * h + j) ^ aswz)]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        a[mt][j] = *reinterpret_cast<const dc::f32x4*>(
-            &(kB ? lds_a1 : lds_a0)[(wm * kW + mt * 32 + r) * kBKd + 4 * ((ks / 4 + 2 * h + j) ^ aswz)]);
-#pragma unroll
-    for (int nt = 0; nt < kMT; ++nt) {
-      const int n = wn * kW + nt * 32 + r;
-#pragma unroll
-      for (int kk = 0; kk < 8; ++kk)
-        b[nt][kk] = (kB ? lds_b1 : lds_b0)[(ks + 8 * h + kk) * T + 4 * ((n >> 2) ^ (8 * h)) + (n & 3)];
-    }
+    for (int kk = 0; kk < 8; ++kk) b[kk] = (kB ? lds_b1 : lds_b0)[(ks + 8 * h + kk) * kT32 + 4 * ((n >> 2) ^ (8 * h)) + (n & 3)];
   };
-  auto mfmas = [&](const dc::f32x4 (&a)[kMT][2], const float (&b)[kMT][8]) __attribute__((always_inline)) {
+  auto mfmas = [&](const dc::f32x4 (&a)[2], const float (&b)[8]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk)
-#pragma unroll
-      for (int mt = 0; mt < kMT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < kMT; ++nt)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mt][kk >> 2][kk & 3], b[nt][kk], acc[mt][nt], 0, 0, 0);
+    for (int kk = 0; kk < 8; ++kk) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[kk >> 2][kk & 3], b[kk], acc, 0, 0, 0);
   };
-  constexpr int kReads = 2 * kMT + 8 * kMT;  // LDS reads per step
   auto interleave_reads = []() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kReads; ++i) {
+    for (int i = 0; i < 10; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // 1 LDS read
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
     }
   };
-  dc::f32x4 fa0[kMT][2], fa1[kMT][2];
-  float fb0[kMT][8], fb1[kMT][8];
+  dc::f32x4 fa0[2], fa1[2];
+  float fb0[8], fb1[8];
   read_frags(std::integral_constant<int, 0>{}, 0, fa0, fb0);
   // Tile KT in LDS buffer BUF = KT % 2 (unrolled by two so buffer offsets are constants; a macro
   // keeps the fragment arrays plain registers). After the last tile the barrier and the reads of
@@ -214,7 +192,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_dma_kernel(const float* 
     interleave_reads();                                                                           \
     __builtin_amdgcn_sched_barrier(0);                                                            \
     dma_barrier(); /* tile KT+1 is in LDS; every wave is done reading buffer BUF */               \
-    if ((KT) + 2 < kt_count) f32_tile_to_lds<T, BUF>(sm, ra, B, N, K, n0, ((KT) + 2) * kBKd, wave, avoff, bvoff); \
+    if ((KT) + 2 < kt_count) f32_tile_to_lds<BUF>(sm, ra, B, N, K, n0, ((KT) + 2) * kBK32, wave, avoff, bvoff); \
     __builtin_amdgcn_sched_barrier(0);                                                            \
     read_frags(std::integral_constant<int, 1 - (BUF)>{}, 0, fa0, fb0);                            \
     mfmas(fa1, fb1);                                                                              \
@@ -227,177 +205,122 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_dma_kernel(const float* 
   }
 #undef DC_F32_TILE
 
-  // acc[mt][nt][v] holds C[row][col], row = 8*(v/4) + 4*h + v%4, col = r (within the 32×32 tile).
+  // acc[v] holds C[row][col], row = 8*(v/4) + 4*h + v%4, col = r (within the wave's 32×32 tile).
+  const int col = n0 + wn * 32 + r;
 #pragma unroll
-  for (int mt = 0; mt < kMT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < kMT; ++nt) {
-      const int col = n0 + wn * kW + nt * 32 + r;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm * kW + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-        C[(size_t)row * N + col] = acc[mt][nt][v];
-      }
-    }
+  for (int v = 0; v < 16; ++v) C[(size_t)(m0 + wm * 32 + 8 * (v >> 2) + 4 * h + (v & 3)) * N + col] = acc[v];
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp32, bounds-checked. T = macro tile; 4 waves as 2×2, each wave (T/2)×(T/2) = (T/64)×(T/64) MFMA
-// 32×32 tiles. The next tile's global loads go to registers before the current tile's MFMAs and are
-// stored to the other LDS buffer afterwards, with B transposed on the way in (Bs[n][k], row pitch
-// BK + 4 floats), so a lane's operands for 8 MFMAs are two contiguous, bank-conflict-free 16-byte
-// LDS reads.
+// fp32, bounds-checked 64×64 tiles, 2×2 waves of 32×32. The next tile's global loads go to registers
+// before the current tile's MFMAs and are stored to the other LDS buffer afterwards, with B
+// transposed on the way in (b[n][k], row pitch 36 floats), so a lane's operands for 8 MFMAs are two
+// contiguous, bank-conflict-free 16-byte LDS reads.
 // ---------------------------------------------------------------------------------------------
-template <int BK, int T>
 struct F32Smem {
-  static constexpr int kPitch = BK + 4;  // floats per LDS row
-  float a[2][T][kPitch];
-  float b[2][T][kPitch];
+  static constexpr int kPitch = kBK32 + 4;  // floats per LDS row
+  float a[2][kT32][kPitch];
+  float b[2][kT32][kPitch];
 };
 
-// Global -> register prefetch for one BK slice. A: (T rows × BK) as float4 slots,
-// slot s -> row s / (BK/4), kq = s % (BK/4). B: (BK × T) as float4 slots, slot s ->
-// nq = s / BK, k = s % BK (a wave covers 16 k-rows × 4 column quads, which spreads the transposed
-// LDS writes over the banks).
-template <int BK, bool CHECKED, int T>
+// Global -> register prefetch for one slice of 32 k. A (64 rows × 32 k) as float4 slots, slot s -> row
+// s / 8, kq = s % 8. B (32 × 64) as float4 slots, slot s -> nq = s / 32, k = s % 32 (a wave covers 32
+// k-rows × 2 column quads, which spreads the transposed LDS writes over the banks).
 struct F32Loader {
-  static constexpr int kASlots = T * BK / 4 / kThreads;
-  static constexpr int kBSlots = T * BK / 4 / kThreads;
-  dc::f32x4 ra[kASlots];
-  dc::f32x4 rb[kBSlots];
+  static constexpr int kSlots = kT32 * kBK32 / 4 / kThreads;
+  dc::f32x4 ra[kSlots];
+  dc::f32x4 rb[kSlots];
+
+  // p[0..4), those elements that are left; zeros where none is (valid false).
+  static __device__ inline dc::f32x4 quad(const float* p, int left, bool valid) {
+    dc::f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (valid) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < left) v[e] = p[e];
+    }
+    return v;
+  }
 
   __device__ inline void load(const float* __restrict__ A, const float* __restrict__ B, int M, int N, int K,
                               int m0, int n0, int k0, int tid) {
 #pragma unroll
-    for (int i = 0; i < kASlots; ++i) {
+    for (int i = 0; i < kSlots; ++i) {
       const int s = tid + i * kThreads;
-      const int row = s / (BK / 4), kq = s % (BK / 4);
-      const int gm = m0 + row, gk = k0 + 4 * kq;
-      if (!CHECKED) {
-        ra[i] = *reinterpret_cast<const dc::f32x4*>(A + (size_t)gm * K + gk);
-      } else {
-        dc::f32x4 v = {0.f, 0.f, 0.f, 0.f};
-        if (gm < M) {
-          const float* p = A + (size_t)gm * K;
-          if (gk + 0 < K) v.x = p[gk + 0];
-          if (gk + 1 < K) v.y = p[gk + 1];
-          if (gk + 2 < K) v.z = p[gk + 2];
-          if (gk + 3 < K) v.w = p[gk + 3];
-        }
-        ra[i] = v;
-      }
+      const int gm = m0 + s / (kBK32 / 4), gk = k0 + 4 * (s % (kBK32 / 4));
+      ra[i] = quad(A + (size_t)gm * K + gk, K - gk, gm < M);
     }
 #pragma unroll
-    for (int i = 0; i < kBSlots; ++i) {
+    for (int i = 0; i < kSlots; ++i) {
       const int s = tid + i * kThreads;
-      const int nq = s / BK, k = s % BK;
-      const int gk = k0 + k, gn = n0 + 4 * nq;
-      if (!CHECKED) {
-        rb[i] = *reinterpret_cast<const dc::f32x4*>(B + (size_t)gk * N + gn);
-      } else {
-        dc::f32x4 v = {0.f, 0.f, 0.f, 0.f};
-        if (gk < K) {
-          const float* p = B + (size_t)gk * N;
-          if (gn + 0 < N) v.x = p[gn + 0];
-          if (gn + 1 < N) v.y = p[gn + 1];
-          if (gn + 2 < N) v.z = p[gn + 2];
-          if (gn + 3 < N) v.w = p[gn + 3];
-        }
-        rb[i] = v;
-      }
+      const int gk = k0 + s % kBK32, gn = n0 + 4 * (s / kBK32);
+      rb[i] = quad(B + (size_t)gk * N + gn, N - gn, gk < K);
     }
   }
 
-  __device__ inline void store(F32Smem<BK, T>& sm, int buf, int tid) {
+  __device__ inline void store(F32Smem& sm, int buf, int tid) {
 #pragma unroll
-    for (int i = 0; i < kASlots; ++i) {
+    for (int i = 0; i < kSlots; ++i) {
       const int s = tid + i * kThreads;
-      const int row = s / (BK / 4), kq = s % (BK / 4);
-      *reinterpret_cast<dc::f32x4*>(&sm.a[buf][row][4 * kq]) = ra[i];
+      *reinterpret_cast<dc::f32x4*>(&sm.a[buf][s / (kBK32 / 4)][4 * (s % (kBK32 / 4))]) = ra[i];
     }
 #pragma unroll
-    for (int i = 0; i < kBSlots; ++i) {
+    for (int i = 0; i < kSlots; ++i) {
       const int s = tid + i * kThreads;
-      const int nq = s / BK, k = s % BK;
-      sm.b[buf][4 * nq + 0][k] = rb[i].x;
-      sm.b[buf][4 * nq + 1][k] = rb[i].y;
-      sm.b[buf][4 * nq + 2][k] = rb[i].z;
-      sm.b[buf][4 * nq + 3][k] = rb[i].w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sm.b[buf][4 * (s / kBK32) + e][s % kBK32] = rb[i][e];
     }
   }
 };
 
-template <int BK, bool CHECKED, int T>
 __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
                                                                float* __restrict__ C, int M, int N, int K, int tiles_m,
                                                                int tiles_n) {
-  constexpr int kW = T / 2, kMT = T / 64;  // wave tile edge, MFMA tiles per wave edge
-  __shared__ F32Smem<BK, T> sm;
+  __shared__ F32Smem sm;
   const TileCoord tc = map_tile(tiles_m, tiles_n);
   if (tc.tm < 0) return;
-  const int m0 = tc.tm * T, n0 = tc.tn * T;
+  const int m0 = tc.tm * kT32, n0 = tc.tn * kT32;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int r = lane & 31, h = lane >> 5;
 
-  f32x16 acc[kMT][kMT];
+  f32x16 acc;
 #pragma unroll
-  for (int i = 0; i < kMT; ++i)
-#pragma unroll
-    for (int j = 0; j < kMT; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
 
-  F32Loader<BK, CHECKED, T> ld;
-  const int kt_count = (K + BK - 1) / BK;
+  F32Loader ld;
+  const int kt_count = (K + kBK32 - 1) / kBK32;
   ld.load(A, B, M, N, K, m0, n0, 0, tid);
   ld.store(sm, 0, tid);
   __syncthreads();
 
   for (int kt = 0; kt < kt_count; ++kt) {
     const int buf = kt & 1;
-    if (kt + 1 < kt_count) ld.load(A, B, M, N, K, m0, n0, (kt + 1) * BK, tid);
+    if (kt + 1 < kt_count) ld.load(A, B, M, N, K, m0, n0, (kt + 1) * kBK32, tid);
 #pragma unroll
-    for (int ks = 0; ks < BK; ks += 16) {
-      dc::f32x4 a[kMT][2], b[kMT][2];
+    for (int ks = 0; ks < kBK32; ks += 16) {
+      dc::f32x4 a[2], b[2];
+      const float *pa = &sm.a[buf][wm * 32 + r][ks + 8 * h], *pb = &sm.b[buf][wn * 32 + r][ks + 8 * h];
 #pragma unroll
-      for (int mt = 0; mt < kMT; ++mt) {
-        const float* p = &sm.a[buf][wm * kW + mt * 32 + r][ks + 8 * h];
-        a[mt][0] = *reinterpret_cast<const dc::f32x4*>(p);
-        a[mt][1] = *reinterpret_cast<const dc::f32x4*>(p + 4);
+      for (int j = 0; j < 2; ++j) {
+        a[j] = *reinterpret_cast<const dc::f32x4*>(pa + 4 * j);
+        b[j] = *reinterpret_cast<const dc::f32x4*>(pb + 4 * j);
       }
 #pragma unroll
-      for (int nt = 0; nt < kMT; ++nt) {
-        const float* p = &sm.b[buf][wn * kW + nt * 32 + r][ks + 8 * h];
-        b[nt][0] = *reinterpret_cast<const dc::f32x4*>(p);
-        b[nt][1] = *reinterpret_cast<const dc::f32x4*>(p + 4);
-      }
-#pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-#pragma unroll
-        for (int mt = 0; mt < kMT; ++mt)
-#pragma unroll
-          for (int nt = 0; nt < kMT; ++nt)
-            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mt][kk >> 2][kk & 3], b[nt][kk >> 2][kk & 3],
-                                                               acc[mt][nt], 0, 0, 0);
-      }
+      for (int kk = 0; kk < 8; ++kk)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[kk >> 2][kk & 3], b[kk >> 2][kk & 3], acc, 0, 0, 0);
     }
     if (kt + 1 < kt_count) ld.store(sm, buf ^ 1, tid);
     __syncthreads();
   }
 
-  // acc[mt][nt][v] holds C[row][col], row = 8*(v/4) + 4*h + v%4, col = r (within the 32×32 tile).
+  // acc[v] holds C[row][col], row = 8*(v/4) + 4*h + v%4, col = r (within the wave's 32×32 tile).
+  const int col = n0 + wn * 32 + r;
 #pragma unroll
-  for (int mt = 0; mt < kMT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < kMT; ++nt) {
-      const int col = n0 + wn * kW + nt * 32 + r;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm * kW + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-        if (!CHECKED || (row < M && col < N)) C[(size_t)row * N + col] = acc[mt][nt][v];
-      }
-    }
+  for (int v = 0; v < 16; ++v) {
+    const int row = m0 + wm * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+    if (row < M && col < N) C[(size_t)row * N + col] = acc[v];
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -435,9 +358,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const float* __re
 //   past N re-read the last ones (their results are not stored); in a last tile of fewer than 64 k
 //   the chunks past K are requested past the buffer range, which loads zeros.
 // - registers (any other shape): 16-byte loads at the elements' own alignment, stored to the same
-//   LDS slots a tile later. A tile past M or N is moved back to end at M or N, so its loads need no
-//   checks (rows and columns that another tile owns are not stored); the last tile of a ragged k,
-//   and matrices smaller than one tile, take element-wise checked loads.
+//   LDS slots a tile later. A tile past N is moved back to end there and rows past M re-read the last
+//   one, so its loads need no checks (rows past M and columns that another tile owns are not stored);
+//   the last tile of a ragged k, and matrices of fewer columns than a tile, take element-wise checked
+//   loads.
 //
 // Pipeline of tile kt (buffer kt & 1): steps 0..2 run their MFMAs with the next step's fragment
 // reads between them; then the tile's one barrier (which also waits for tile kt+1's loads, issued
@@ -1283,8 +1207,6 @@ __global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float* __restric
   }
 }
 
-constexpr int kBKf32 = 32;
-
 dim3 tile_grid(int tiles_m, int tiles_n, int threads) {
   const dc::GemmGrid g = dc::gemm_grid((int64_t)tiles_m * tiles_n, threads);
   return dim3((unsigned)g.x, (unsigned)g.rows);
@@ -1324,14 +1246,14 @@ DC_HIP_API int32_t dc_hip_gemm_f32(dc_hip_ctx* ctx, const float* a, const float*
   if (!c || (k > 0 && (!a || !b))) return DC_ERR_INVALID_ARGUMENT;
   DC_CTX_ENTER(ctx);
   if (k == 0) return dc::zero_async(ctx, c, (size_t)(m * n) * sizeof(float));
-  const int tiles_m = (int)((m + 63) / 64), tiles_n = (int)((n + 63) / 64);
+  const int tiles_m = (int)((m + kT32 - 1) / kT32), tiles_n = (int)((n + kT32 - 1) / kT32);
   switch (dc::f32_gemm_kernel(m, n, k, dc::aligned16(a) && dc::aligned16(b), std::max(1, ctx->cu_count))) {
     case dc::F32Gemm::kDma64:
-      gemm_f32_dma_kernel<64><<<tile_grid(tiles_m, tiles_n, kThreads), kThreads, 0, ctx->stream>>>(
-          a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
+      gemm_f32_dma_kernel<<<tile_grid(tiles_m, tiles_n, kThreads), kThreads, 0, ctx->stream>>>(a, b, c, (int)n, (int)k,
+                                                                                               tiles_m, tiles_n);
       break;
     case dc::F32Gemm::kChecked64:
-      gemm_f32_kernel<kBKf32, true, 64><<<tile_grid(tiles_m, tiles_n, kThreads), kThreads, 0, ctx->stream>>>(
+      gemm_f32_kernel<<<tile_grid(tiles_m, tiles_n, kThreads), kThreads, 0, ctx->stream>>>(
           a, b, c, (int)m, (int)n, (int)k, tiles_m, tiles_n);
       break;
     case dc::F32Gemm::kSplit256x128: launch_split<256, 128, 4, 2, 1, 1>(ctx, a, b, c, m, n, k); break;

@@ -370,12 +370,6 @@ __device__ inline int first_fault(const Faults& f, bool* overflow) {
   return j;
 }
 
-// ---- affine-chain fast path -------------------------------------------------------------------
-// Chains whose every stage is `Where(x <cmp> c)` or `Select(x * a + b)` (also x*a, x+b, x-b) are
-// lowered to a stage table and run without the interpreter's scratch registers, which lets more
-// tiles be resident. Each stage rounds exactly as the interpreter does (x*a, then +b).
-constexpr int kMaxAffineStages = 8;
-enum AffineKind : uint8_t { kStageFilter = 0, kStageMap = 1 };
 // ---- one comparison pair, then a short polynomial ------------------------------------------------
 // Programs `Where(y <cmp> c [&&/|| y <cmp> c']).Select(x => three steps at most of + - * with a
 // constant or x)`, either part optional, y = x or (int32) x % constant. The interpreter spends most of
@@ -441,6 +435,12 @@ __device__ __attribute__((always_inline)) inline float poly_map(const PolyChain&
   return __builtin_bit_cast(float, v);
 }
 
+// ---- affine-chain fast path -------------------------------------------------------------------
+// Chains whose every stage is `Where(x <cmp> c)` or `Select(x * a + b)` (also x*a, x+b, x-b) are
+// lowered to a stage table and run without the interpreter's scratch registers, which lets more
+// tiles be resident. Each stage rounds exactly as the interpreter does (x*a, then +b).
+constexpr int kMaxAffineStages = 8;
+enum AffineKind : uint8_t { kStageFilter = 0, kStageMap = 1 };
 // Fields are 32-bit so the kernel reads them with scalar loads (no scalar byte loads on gfx950).
 struct AffineChain {
   int32_t n_stages;

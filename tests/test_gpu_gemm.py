@@ -70,8 +70,8 @@ def test_gemm_f32_full_tiles(ctx, shape):
     check_rows(c, a, b, np.arange(m))
 
 
-# Full-tile shapes run the direct-to-LDS kernel (64-tiles below 2 * CUs 128-tiles, else 128-tiles);
-# these cover one, two and an odd number of 32-wide k tiles for both tile sizes.
+# Full 64-tiles on the fp32 instructions (direct-to-LDS loads): one, two and an odd number of 32-wide k
+# tiles, few and many tiles.
 @pytest.mark.parametrize("shape", [(128, 128, 32), (192, 320, 96), (256, 64, 64), (4096, 2048, 32),
                                    (2048, 4096, 64), (4096, 2048, 96)])
 def test_gemm_f32_k_tile_counts(ctx, shape):
@@ -90,8 +90,8 @@ def test_gemm_f32_reference_case_vs_fp32_loop(ctx):
     assert np.max(np.abs(c - expected)) <= 1e-3
 
 
-# Shapes with fewer than 2 * CUs tiles of 128x128 run 64x64 tiles; (4000, 2100, 37) has 544 of them
-# and takes the bounds-checked 128x128 kernel.
+# The bounds-checked 64x64 tiles (fewer than 64 columns, k of 16 or less), and ragged split tiles: 64 with
+# one and two k groups, 128 for (4000, 2100, 37).
 @pytest.mark.parametrize("shape", [(1, 1, 1), (3, 5, 7), (100, 37, 53), (129, 130, 131), (257, 64, 1000),
                                    (4000, 2100, 37)])
 def test_gemm_f32_ragged(ctx, shape):
@@ -130,9 +130,8 @@ def test_gemm_f32_large_sampled(ctx, n):
     freivalds(c, a, b)
 
 
-# (256-multiples of m and n with k a multiple of 64 take the 256x256-tile kernel, which reads
-# row-major B through transposing LDS reads, with 1, 2, 3, 6 and more 64-wide k tiles; the other
-# shapes the 128x128 kernels)
+# (64-tiles with one and two k groups, over 1, 2, 3, 6 and more 64-wide k tiles; B through transposing LDS
+# reads. (100, 37, 53): loads through registers. The others: test_gemm_bf16_ragged_tiles.)
 @pytest.mark.parametrize("shape", [(128, 128, 64), (512, 768, 384), (100, 37, 53), (256, 256, 64),
                                    (1024, 512, 1024), (768, 1280, 192), (256, 512, 4096), (384, 256, 64),
                                    (512, 256, 128)])
@@ -171,11 +170,12 @@ def test_convert_f32_to_bf16_bit_exact(ctx):
     ctx.free(o)
 
 
-# One shape or two per tile choice of the bf16 dispatch (on 256 CUs), each with ragged rows, columns
-# and a last k tile that is not whole. 16-byte rows: 256-tiles, 128-tiles (two), 128-tiles with two k
+# One shape or more per tile choice of the bf16 dispatch (on 256 CUs), with ragged rows, columns and a
+# last k tile that is not whole. 16-byte rows: 256-tiles of one to four k tiles, 128-tiles (two), 128-tiles with two k
 # groups, 64-tiles with one, two and four; other rows: 128-tiles, 64-tiles with one and four k groups,
 # fewer columns than a tile. (host_tests.cpp checks that each shape takes the kernel it is here for.)
-@pytest.mark.parametrize("shape", [(2824, 3080, 72), (4104, 4360, 136), (2200, 2056, 200), (1800, 1912, 136), (200, 264, 200), (8, 8, 8),
+@pytest.mark.parametrize("shape", [(4096, 4096, 64), (2824, 3080, 72), (2816, 3072, 192), (2824, 3080, 200), (4104, 4360, 136),
+                                   (2200, 2056, 200), (1800, 1912, 136), (200, 264, 200), (8, 8, 8),
                                    (456, 520, 520), (72, 136, 2120), (1799, 1911, 137), (63, 65, 129), (300, 50, 70),
                                    (129, 131, 1001), (70, 9, 64)])
 def test_gemm_bf16_ragged_tiles(ctx, shape):
