@@ -623,28 +623,57 @@ POLY_STEPS = [None, [], [(MUL, SRC_ELEM, 0)], [(MUL, SRC_ELEM, 0), (ADD, SRC_ELE
               [(SUB, SRC_ELEM, 0), (ADD, SRC_IMM, 3.0), (MUL, SRC_ELEM, 0)], [(SUB, SRC_IMM, 0.1), (MUL, SRC_IMM, -3.0)]]
 
 
-@pytest.mark.parametrize("cmp", [None, CMP_GT, CMP_GE, CMP_LT, CMP_LE, CMP_EQ, CMP_NE])
-@pytest.mark.parametrize("second", range(len(POLY_SECOND)))
+POLY_FILTERS = [(None, 0)] + [(cmp, second) for cmp in (CMP_GT, CMP_GE, CMP_LT, CMP_LE, CMP_EQ, CMP_NE)
+                              for second in range(len(POLY_SECOND))]
+
+
+def poly_program(cmp, second, steps):
+    """Where(x <cmp> 0.25 [second comparison]).Select(steps), either part optional."""
+    code = []
+    if cmp is not None:
+        code += [(LOAD, SRC_ELEM, 0), (cmp, SRC_IMM, 0.25)]
+        if POLY_SECOND[second]:
+            mode, op, imm = POLY_SECOND[second]
+            code.append((op, SRC_IMM, imm, mode))
+        code.append((FILTER, SRC_IMM, 0))
+    if steps is not None:
+        code += [(LOAD, SRC_ELEM, 0)] + steps + [(MAP, SRC_IMM, 0)]
+    return LinqChain.assemble(code) if code else None
+
+
+@pytest.mark.parametrize("cmp,second", POLY_FILTERS)
 def test_poly_programs_match_interpreter(ctx, cmp, second):
-    if cmp is None and second:
-        pytest.skip("a second comparison needs a first")
     x = oracle.gen_uniform_f32(3 * RR_TILE + 7, 900 + second, 0)
     x[::11] = np.resize(np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-40, 0.25, -0.25, 0.5, -0.5], np.float32), x[::11].size)
     for i, steps in enumerate(POLY_STEPS):
-        code = []
-        if cmp is not None:
-            code += [(LOAD, SRC_ELEM, 0), (cmp, SRC_IMM, 0.25)]
-            if POLY_SECOND[second]:
-                mode, op, imm = POLY_SECOND[second]
-                code.append((op, SRC_IMM, imm, mode))
-            code.append((FILTER, SRC_IMM, 0))
-        if steps is not None:
-            code += [(LOAD, SRC_ELEM, 0)] + steps + [(MAP, SRC_IMM, 0)]
-        if not code:
+        prog = poly_program(cmp, second, steps)
+        if prog is None:
             continue
-        prog = LinqChain.assemble(code)
         assert same_floats(run_to_array(ctx, prog, x, offset=i % 4), oracle.linq_where_select(prog, x))
         fin = x[np.isfinite(x)]
         got, cnt = run_sum(ctx, prog, fin)
         _, sd, rc = oracle.linq_where_select_sum(prog, fin)
         assert cnt == rc and abs(got - sd) <= 1e-5 * math.log2(fin.size) * max(abs(sd), 1.0)
+        # the other reductions of the same kernel: the element picked, and the in-order fold
+        for ops, ref_of in ((MINMAX, oracle.linq_where_select_minmax), (FOLDS, oracle.linq_where_select_fold)):
+            for name, op in ops:
+                for data in (x, fin):
+                    got, cnt = run_minmax(ctx, prog, data, op, offset=i % 4)
+                    ref, rcnt = ref_of(prog, data, name)
+                    assert cnt == rcnt, (name, i)
+                    if rcnt:
+                        assert same_floats(np.array([got]), np.array([ref])), (name, i, got, ref)
+
+
+@pytest.mark.parametrize("offset", range(4))
+def test_poly_programs_over_full_rounds(ctx, offset):
+    """The round-robin grid's main loop (loads four rounds ahead, the ring, the delayed write that maps
+    the kept elements, the drain) over four full rounds and a ragged fifth: programs that keep half of
+    the elements, all of them (the ring fills up) and almost none."""
+    x = _salted_input(rr_min_n() + 3 * RR_TILE + 5, 77 + offset)
+    quadratic = [(MUL, SRC_ELEM, 0), (ADD, SRC_ELEM, 0)]
+    for where in ([(CMP_GT, SRC_IMM, -0.5), (CMP_LT, SRC_IMM, 0.5, hip.CMP_AND)], None,
+                  [(CMP_LT, SRC_IMM, 0.0), (CMP_GE, SRC_IMM, 0.0, hip.CMP_OR)], [(CMP_GT, SRC_IMM, 0.999), (CMP_EQ, SRC_IMM, 0.25, hip.CMP_OR)]):
+        code = [(LOAD, SRC_ELEM, 0)] + where + [(FILTER, SRC_IMM, 0)] if where else []
+        prog = LinqChain.assemble(code + [(LOAD, SRC_ELEM, 0)] + quadratic + [(MAP, SRC_IMM, 0)])
+        assert same_floats(run_to_array_checked(ctx, prog, x, hip.STRATEGY_ROUNDS, offset), oracle.linq_where_select(prog, x))

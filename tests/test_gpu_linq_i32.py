@@ -376,3 +376,24 @@ def test_poly_programs_match_oracle(ctx, rem, cmp):
         ch = hip.LinqChain.assemble(code, int32=True)
         got = run_to_array(ctx, ch, x, offset=i % 4)[0]
         assert np.array_equal(got, oracle.linq_where_select_i32(ch, x)[0])
+
+
+# The round-robin grid's main loop (four full rounds and a ragged one) with programs of the
+# comparison-pair-and-polynomial form, with and without a remainder, keeping half, all and few elements,
+# and with one that is interpreted without save registers: every element against the oracle.
+@pytest.mark.parametrize("offset", range(4))
+def test_programs_over_full_rounds(ctx, offset):
+    x = oracle.gen_uniform_i32(4 * min(hip.device_info(0).compute_units, 256) * 8192 + 24_581, 58 + offset, 1, -1000, 1000)
+    x[::13] = np.resize(np.array([0, 1, -1, I32_MAX, I32_MIN, I32_MIN + 1], np.int32), x[::13].size)
+    load, square = (LOAD, SRC_ELEM, 0), [(LOAD, SRC_ELEM, 0), (MUL, SRC_ELEM, 0), (ADD, SRC_IMM, 3), (MAP, SRC_IMM, 0)]
+    programs = [GUARDED_DIV, chain(square)]
+    for where in ([(CMP_GT, SRC_IMM, 0)], [(CMP_LT, SRC_IMM, 0), (hip.CMP_GE, SRC_IMM, 0, hip.CMP_OR)],
+                  [(REM, SRC_IMM, -7), (CMP_NE, SRC_IMM, 0)], [(REM, SRC_IMM, 1000), (CMP_EQ, SRC_IMM, 999)]):
+        programs.append(chain([load] + where + [(FILTER, SRC_IMM, 0)] + square))
+    d, src = put(ctx, x, offset)
+    assert ctx.to_array_strategy(src, x.size) == hip.STRATEGY_ROUNDS
+    ctx.free(d)
+    for i, ch in enumerate(programs):
+        got, k, f = run_to_array(ctx, ch, x, offset)
+        ref, rf = oracle.linq_where_select_i32(ch, x)
+        assert f == rf == -1 and k == ref.size and np.array_equal(got, ref), i
