@@ -46,17 +46,15 @@ constexpr int kThreads = 256;
 constexpr int kGroupM = 8;
 
 struct TileCoord {
-  int tm, tn;  // tm < 0: none (past the last tile, in a grid of more than one row)
+  int tm, tn;
 };
 
 __device__ inline TileCoord map_tile(int tiles_m, int tiles_n) {
   const int total = tiles_m * tiles_n;
-  int b = blockIdx.x;
-  if (blockIdx.y != 0) {  // (dc::gemm_grid)
-    b += (int)(blockIdx.y * gridDim.x);
-    if (b >= total) return TileCoord{-1, 0};
-  }
-  int t = (total % 8 == 0) ? (b % 8) * (total / 8) + b / 8 : b;
+  // (dc::gemm_grid's rows; workgroups past the last tile form that one too: an early exit here costs
+  // every launch 0.1-0.2 us)
+  const int b = min((int)(blockIdx.x + (blockIdx.y << dc::kGemmGridRowBits)), total - 1);
+  const int t = (total % 8 == 0) ? (b % 8) * (total / 8) + b / 8 : b;
   const int group = kGroupM * tiles_n;
   const int g = t / group;
   const int first_m = g * kGroupM;
@@ -128,7 +126,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_dma_kernel(const float* 
   __shared__ __align__(16) float lds_a0[kT32 * kBK32], lds_a1[kT32 * kBK32], lds_b0[kBK32 * kT32], lds_b1[kBK32 * kT32];
   const F32DmaSmem sm{{lds_a0, lds_a1}, {lds_b0, lds_b1}};
   const TileCoord tc = map_tile(tiles_m, tiles_n);
-  if (tc.tm < 0) return;
   const int m0 = tc.tm * kT32, n0 = tc.tn * kT32;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -278,7 +275,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const float* __re
                                                                int tiles_n) {
   __shared__ F32Smem sm;
   const TileCoord tc = map_tile(tiles_m, tiles_n);
-  if (tc.tm < 0) return;
   const int m0 = tc.tm * kT32, n0 = tc.tn * kT32;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -421,7 +417,6 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
   using Smem = Bf16Smem<TM, TN>;
   __shared__ __align__(16) Smem sms[KS];
   const TileCoord tc = map_tile(tiles_m, tiles_n);
-  if (tc.tm < 0) return;
   const int m0 = tc.tm * TM;
   // (register loader: the last tile ends at N where N holds a whole tile)
   const int n0 = kDma || N < TN ? tc.tn * TN : min(tc.tn * TN, N - TN);
@@ -864,7 +859,6 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
   __shared__ int s_redo, s_tiny, s_low;
   __shared__ uint32_t s_seen, s_big;
   const TileCoord tc = map_tile(tiles_m, tiles_n);
-  if (tc.tm < 0) return;
   const int m0 = tc.tm * TM;
   const int n0 = min(tc.tn * TN, N - TN);  // the last tile ends at N (N >= TN, by the host)
   const int tid = threadIdx.x, lane = tid & 63, gwave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -6,14 +6,17 @@
 
 namespace dc {
 
-// The grid of `tiles` workgroups: rows of `x` of them, more than one row where a single one would have
-// more work items than a launch takes in a dimension (2^32 - 1); the last row may be partly empty.
+// The grid of `tiles` workgroups: one row of them, or rows of kGemmGridRow where a single one would have
+// more work items than a launch takes in a dimension (2^32 - 1); the last row may be partly empty. (A
+// fixed row, so that the kernels need no launch dimensions: those cost 0.2 us a launch.)
+constexpr int kGemmGridRowBits = 20;
+constexpr int64_t kGemmGridRow = int64_t(1) << kGemmGridRowBits;
 struct GemmGrid {
   int64_t x, rows;
 };
 inline GemmGrid gemm_grid(int64_t tiles, int64_t threads) {
-  const int64_t most = (int64_t)UINT32_MAX / threads, rows = (tiles + most - 1) / most;
-  return {(tiles + rows - 1) / rows, rows};
+  if (tiles * threads <= (int64_t)UINT32_MAX) return {tiles, 1};
+  return {kGemmGridRow, (tiles + kGemmGridRow - 1) >> kGemmGridRowBits};
 }
 
 // fp32: "Split": the bf16 matrix cores, by tile (rows x columns) and k groups; the others the fp32
