@@ -654,8 +654,8 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
 // seven small products stand in accumulators of their own and are added once, at the end: an
 // instruction's sum may be off by nearly an ulp (these matrix cores cut the addends at half an ulp of
 // the largest before they round), which matters 2^-7 times less in the small sums, and the large ones
-// are rounded once per 16 products where the fp32 instructions round each. So the result is closer to
-// the float64 product than theirs: relative error with normal inputs 8192^3 5.7e-7 against 1.62e-6,
+// are rounded once per 8 products (by the errors) where the fp32 instructions round each. So the result
+// is closer to the float64 product than theirs: relative error with normal inputs 8192^3 5.7e-7 against 1.62e-6,
 // 1537×2049×1023 1.3e-7 against 5.7e-7; a sum of one term is within 0.62 ulp (0.50). (All in one
 // accumulator, 256×256 tiles: 5.74 ms at 8192^3, 1.44e-6, one term up to an ulp off. Six products,
 // without a1 b2 and a2 b1: 4.6 ms, each product off by up to 2^-24 of it, one term up to 1.5 ulp.)

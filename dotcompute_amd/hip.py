@@ -487,9 +487,11 @@ class Context:
               "dc_hip_linq_where_select_minmax_i32")
 
     def gemm_f32(self, a: DeviceArray, b: DeviceArray, c: DeviceArray, m: int, n: int, k: int) -> None:
+        """C = A B in fp32: each product within 2^-34 of it, fp32 sums (include/dotcompute_hip.h)."""
         check(load().dc_hip_gemm_f32(self.handle, a.ptr, b.ptr, c.ptr, m, n, k), "dc_hip_gemm_f32")
 
     def gemm_bf16(self, a: DeviceArray, b: DeviceArray, c: DeviceArray, m: int, n: int, k: int) -> None:
+        """C = A B from bf16 bit patterns, fp32 sums and result."""
         check(load().dc_hip_gemm_bf16(self.handle, a.ptr, b.ptr, c.ptr, m, n, k), "dc_hip_gemm_bf16")
 
     def convert_f32_to_bf16(self, x: DeviceArray, out: DeviceArray, n: int | None = None) -> None:
