@@ -691,6 +691,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
 //   (as gemm_bf16_kernel).
 // ---------------------------------------------------------------------------------------------
 constexpr float kSplitMin = 0x1p-102f;
+constexpr int kSplitMinExp = -101;             // its exponent as split_quad counts
 constexpr float kSplitMax = 0x1.fefffep127f;  // the largest magnitude that does not round to infinity in bf16
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -703,15 +704,15 @@ __device__ __attribute__((always_inline)) inline void for_each_index(F&& f, std:
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-// The three bf16 pieces of four values, packed; *big becomes the largest 2|x| (as bits) seen, *tiny the
-// smallest less 1 (all ones for x = 0).
-__device__ inline void split_quad(dc::f32x4 x, u32x2 (&piece)[3], uint32_t* big, uint32_t* tiny) {
+// The three bf16 pieces of four values, packed; *big and *tiny become the largest and smallest exponent
+// seen (|x| in [2^(e-1), 2^e); 0 for zeros, infinities and NaN, which neither reads amiss: see below).
+__device__ inline void split_quad(dc::f32x4 x, u32x2 (&piece)[3], int* big, int* tiny) {
   f32x2 v[2] = {{x.x, x.y}, {x.z, x.w}};
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const uint32_t u0 = __builtin_bit_cast(uint32_t, v[i].x) << 1, u1 = __builtin_bit_cast(uint32_t, v[i].y) << 1;
-    *big = max(*big, max(u0, u1));
-    *tiny = min(*tiny, min(u0 - 1u, u1 - 1u));
+    const int e0 = __builtin_amdgcn_frexp_expf(v[i].x), e1 = __builtin_amdgcn_frexp_expf(v[i].y);
+    *big = max(*big, max(e0, e1));
+    *tiny = min(*tiny, min(e0, e1));
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v[i], bf16x2));
@@ -856,8 +857,8 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
   constexpr int kA = TM * 4 / kT, kB = TN * 4 / kT;  // quads per thread and k tile
   using Smem = SplitSmem<TM, TN>;
   __shared__ __align__(16) Smem sms[KS];
-  __shared__ int s_redo, s_tiny, s_low;
-  __shared__ uint32_t s_seen, s_big;
+  __shared__ int s_redo, s_tiny, s_low, s_big;
+  __shared__ uint32_t s_seen;
   const TileCoord tc = map_tile(tiles_m, tiles_n);
   const int m0 = tc.tm * TM;
   const int n0 = min(tc.tn * TN, N - TN);  // the last tile ends at N (N >= TN, by the host)
@@ -884,7 +885,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
     wb[i] = (uint32_t)(krow * TN + 32 * ((nq >> 3) ^ bswz(krow)) + 4 * (nq & 7));
   }
   dc::f32x4 sa[D][kA], sb[D][kB];  // D tiles of elements in flight
-  uint32_t big = 0, tiny = 0xFFFFFFFFu;  // over the lane's elements: see split_quad
+  int big = -200, tiny = 0;  // over the lane's elements: see split_quad
   // The group's k tile KT, every element of which exists.
   auto load_tile = [&](int KT, dc::f32x4 (&qa)[kA], dc::f32x4 (&qb)[kB]) __attribute__((always_inline)) {
     const int k0 = (KT * KS + group) * kBK;
@@ -1010,7 +1011,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  if (tid == 0) s_redo = s_tiny = s_low = s_seen = s_big = 0;
+  if (tid == 0) s_redo = s_tiny = s_low = s_seen = 0, s_big = -200;
   constexpr std::integral_constant<int, 0> kBuf0{};
   constexpr std::integral_constant<int, 1> kBuf1{};
   static_assert(D == 1 || D == 2, "the loop is unrolled by two");
@@ -1075,7 +1076,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
     } while (p + 1 < kt_count);
     if (p < kt_count) one(p, kBuf0);
   }
-  if (tiny < kTinyBits) s_tiny = 1;
+  if (tiny < kSplitMinExp) s_tiny = 1;
 #pragma unroll
   for (int i = 0; i < kMT * kNT; ++i)
 #pragma unroll
@@ -1105,14 +1106,14 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (KS == 1 && WM * WN == 4 ? 2 : 1
   static_assert(sizeof(Smem) >= 2 * (TM + TN) * sizeof(uint32_t), "the rows' and columns' figures fit in the buffers");
   constexpr float kLost = 0x1p-102f;
   bool scan = s_tiny != 0 && !early;  // uniform, as all of this
-  if (scan) {  // unless every sum stands whatever its row and column hold
-    atomicMax(&s_big, big >> 1);
+  if (scan) {  // unless every sum stands whatever its row and column hold (their infinities and NaN aside:
+               // no sum that those reach is finite)
+    atomicMax(&s_big, big);
     __syncthreads();
-    const float least = __builtin_bit_cast(float, s_big) * 2.0f * ((float)K * kLost);
+    const float least = __builtin_ldexpf(2.0f * (float)K * kLost, s_big);
     bool low = false;
 #pragma unroll
-    for (int i = 0; i < kMT * kNT * 16; ++i)
-      low |= !(__builtin_fabsf(acc[i / 16 / kNT][i / 16 % kNT][i % 16]) >= least);  // (NaN: not known to)
+    for (int i = 0; i < kMT * kNT * 16; ++i) low |= __builtin_fabsf(acc[i / 16 / kNT][i / 16 % kNT][i % 16]) < least;
     if (group == 0 && low) s_low = 1;
     __syncthreads();
     scan = s_low != 0;

@@ -328,19 +328,29 @@ def test_gemm_f32_exceptional_values_stay_in_their_rows_and_columns(ctx, shape):
 @pytest.mark.parametrize("shape", F32_KERNELS)
 def test_gemm_f32_values_whose_pieces_are_lost(ctx, shape):
     """Values near 2^-130 times ones near 2^100: their bf16 pieces would be off by up to 2^-134, a
-    sixteenth of the value. All of A, all of B, one row among ordinary ones, and every third value of it."""
+    sixteenth of the value. All of A, all of B, one row among ordinary ones (with a NaN in a column of B
+    too), and the values at every fourth place of a row of A or a column of B, the rest of it zero."""
     m, n, k = shape
     a, b = make_inputs(m, n, k)
     small, large = np.float32(2.0 ** -130), np.float32(2.0 ** 100)
-    row, third = a * np.float32(2.0 ** -100), a * np.float32(2.0 ** -100)
+    cases = [(a * small, b * large), (a * large, b * small)]
+    row, nan = a * np.float32(2.0 ** -60), b * large
     row[m // 2] = a[m // 2] * small
-    third[m // 2, ::3] = a[m // 2, ::3] * small
-    third[m // 2, 1::3] = third[m // 2, 2::3] = 0
-    for x, y in ((a * small, b * large), (a * large, b * small), (row, b * large), (third, b * large)):
+    nan[k - 1, 4] = np.nan
+    cases += [(row, b * large), (row, nan)]
+    for place in range(4):
+        row, col = a * np.float32(2.0 ** -60), b * np.float32(2.0 ** -60)
+        row[m // 2] = 0
+        row[m // 2, place::4] = a[m // 2, place::4] * small
+        # (four k of A are one load, and four columns of B)
+        col[:, n // 8 * 4 + place] = b[:, n // 8 * 4 + place] * small
+        cases += [(row, b * large), (a * large, col)]
+    for x, y in cases:
         got = run_gemm(ctx, x, y)
         x64, y64 = x.astype(np.float64), y.astype(np.float64)
         # (the float32 product's error, as in the other tests: each of k additions within one ulp)
-        assert np.all(np.abs(got - x64 @ y64) <= (k + 1) * 2.0 ** -23 * (np.abs(x64) @ np.abs(y64)))
+        err, bound = np.abs(got - x64 @ y64), (k + 1) * 2.0 ** -23 * (np.abs(x64) @ np.abs(y64))
+        assert np.all((err <= bound) | np.isnan(bound))
 
 
 @pytest.mark.slow
