@@ -322,7 +322,7 @@ typedef struct dc_linq_instr {
 /* dc_linq_chain.flags bits. DC_LINQ_FLAG_ORDERED_GRID: run a ToArray on the ticket-ordered lookback
  * grid even where the resident grid would be chosen (the retry after a resident grid gave up).
  * DC_LINQ_FLAG_INTERPRET: never compile the program at run time (see dc_linq_chain_compile); run it
- * on the prebuilt interpreter kernels. */
+ * on the prebuilt kernels. */
 #define DC_LINQ_FLAG_ORDERED_GRID 1
 #define DC_LINQ_FLAG_INTERPRET 2
 
@@ -344,7 +344,8 @@ DC_HIP_API int32_t dc_linq_chain_validate_i32(const dc_linq_chain* chain);
  * source feeds the interpreter's own instruction semantics the program as constants. The library
  * builds and caches such kernels (once per process, device, element type and program) for inputs
  * of at least DC_LINQ_COMPILE_MIN_ELEMENTS, but the ToArray entry points do not launch them at
- * present: every program runs on the prebuilt interpreter kernels, and dc_hip_linq_compile_stats
+ * present: every program runs on a prebuilt kernel (the interpreter, or one for affine chains or for a
+ * comparison pair and a short polynomial, with the interpreter's results), and dc_hip_linq_compile_stats
  * reports no compiled launches. DC_LINQ_FLAG_INTERPRET (accepted on every chain) opts a chain
  * out of compilation. */
 #define DC_LINQ_COMPILE_MIN_ELEMENTS (1 << 22)
