@@ -655,9 +655,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS, (WM * WN == 8 ? 1 : 2)) void gem
 // instruction's sum may be off by nearly an ulp (these matrix cores cut the addends at half an ulp of
 // the largest before they round), which matters 2^-7 times less in the small sums, and the large ones
 // are rounded once per 8 products (by the errors) where the fp32 instructions round each. So the result
-// is closer to the float64 product than theirs: relative error with normal inputs 8192^3 5.7e-7 against 1.62e-6,
-// 1537×2049×1023 1.3e-7 against 5.7e-7; a sum of one term is within 0.62 ulp (0.50). (All in one
-// accumulator, 256×256 tiles: 5.74 ms at 8192^3, 1.44e-6, one term up to an ulp off. Six products,
+// is closer to the float64 product than theirs: relative error with normal inputs 5.7e-7 against 1.62e-6
+// at 8192^3, 1.3e-7 against 5.7e-7 at 1537×2049×1023; a sum of one term is within 0.62 ulp (0.50). (All
+// in one accumulator, 256×256 tiles: 5.74 ms at 8192^3, 1.44e-6, one term up to an ulp off. Six products,
 // without a1 b2 and a2 b1: 4.6 ms, each product off by up to 2^-24 of it, one term up to 1.5 ulp.)
 // 8 bf16 products cost half of one fp32 product on this chip's matrix cores. Measured against the
 // kernels on the fp32 instructions: 8192^3 7.30 -> 6.02 ms (183 TFLOP/s where those instructions peak
